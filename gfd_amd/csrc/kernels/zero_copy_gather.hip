@@ -131,11 +131,14 @@ __global__ __launch_bounds__(kBlock) void zc_scatter_tokens(const uint64_t* __re
 }
 
 // Generic SG list: any sizes, any (disjoint) destinations, same batching.
-// The sizes are in the table, which the host does not read, so a short list
-// is split by count instead: each entry is cut into `pieces` slices of
-// ceil(size / pieces) bytes rounded up to 16 (keeping the entry's alignment;
-// the last slice takes the rest and slices past the end are empty), and
-// unit u is slice u % pieces of entry u / pieces.
+// The sizes are in the table, which the host does not read, so a list of few
+// entries is split by count instead: each entry is cut into `pieces` slices
+// of ceil(size / pieces) bytes rounded up to 16 (the last slice takes the rest
+// and slices past the end are empty), and unit u is slice u % pieces of entry
+// u / pieces.  Wave w then takes units w, w + waves, ...: slices of different
+// entries, so unequal entries still give every wave about the same bytes.
+// Whole entries (pieces = 1) go to the waves in runs, which read the table in
+// whole cache lines.
 template <bool kLds>
 __global__ __launch_bounds__(kBlock) void zc_gather_sg(const gfd_sg_entry* __restrict__ entries, uint32_t count,
                                                        uint32_t pieces, uint32_t per_wave, int unroll,
@@ -143,17 +146,19 @@ __global__ __launch_bounds__(kBlock) void zc_gather_sg(const gfd_sg_entry* __res
     __shared__ BatchLds lds[kWavesPerBlock];
     __shared__ gfd::wave::vec4u stage[kLds ? kWavesPerBlock : 1][kLds ? kStageVecs : 1];
     const uint32_t lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    const uint64_t wave = (uint64_t)blockIdx.x * kWavesPerBlock + wid;
-    const uint64_t stride = (uint64_t)gridDim.x * kWavesPerBlock * per_wave;
-    const uint64_t units = (uint64_t)count * pieces;
-    for (uint64_t first = wave * per_wave; first < units; first += stride) {
-        const uint32_t nb = (uint32_t)min((uint64_t)per_wave, units - first);
+    const uint32_t wave = blockIdx.x * kWavesPerBlock + wid, waves = gridDim.x * kWavesPerBlock;
+    // The host launches ceil(units / per_wave) waves or more: one batch each.
+    const uint64_t u = pieces > 1 ? (uint64_t)lane * waves + wave : (uint64_t)wave * per_wave + lane;
+    const bool has = lane < per_wave && u < (uint64_t)count * pieces;
+    const uint32_t nb = (uint32_t)__popcll(__ballot(has));  // the lanes that have one come first
+    if (nb) {
         uint64_t md = 0, ms = 0, mn = 0;
-        if (lane < nb) {
-            const uint64_t u = first + lane;
-            const gfd_sg_entry e = entries[u / pieces];
-            const uint64_t step = ((e.size + pieces - 1) / pieces + 15) & ~15ull;
-            const uint64_t off = min((u % pieces) * step, e.size);
+        if (has) {
+            const uint32_t i = pieces > 1 ? (uint32_t)u / pieces : (uint32_t)u;
+            const uint64_t k = u - (uint64_t)i * pieces;
+            const gfd_sg_entry e = entries[i];
+            const uint64_t step = pieces > 1 ? ((e.size + pieces - 1) / pieces + 15) & ~15ull : e.size;
+            const uint64_t off = min(k * step, e.size);
             md = e.dst + off;
             ms = e.src + off;
             mn = min(step, e.size - off);
@@ -264,17 +269,28 @@ int launch_scatter_tokens(const uint64_t* dst_addrs, const void* src, uint32_t t
 // Waves a short list is aimed at (GFD_ZC_WAVES, else the minimum grid).
 int short_list_waves() { return std::max(4, env_int(kGatherShape.waves_env, kGatherShape.min_waves)); }
 
-// slice: the table is the caller's list as it is, so a list of at most half
-// the target waves' entries gets target / count waves per entry (slices of a
-// small entry may be empty).  Without it, each record is one wave's work (the
-// caller has cut the list into pieces already).
+// Entry lists of unknown sizes: 256 waves (U = 4: 1 MiB outstanding), and
+// lists of at most half of kSgUnits entries cut into kSgUnits / count slices
+// each.  Measured on MI355X, against one wave per entry (two or more for at
+// most 32 entries) on 64 waves: 48 entries of up to 300 KB 154 -> 141 us, 64
+// of up to 1 MiB 655 -> 614 us, 256 of up to 64 KiB 176 -> 156 us, 100 of up
+// to 64 KiB 76 -> 64 us; 2000 of up to 30 KB 557 -> 543 us by the waves
+// alone.  512 units leave 3% more at 64 entries, 2048 and 4096 cost 5-15% on
+// a single 1 MiB entry; 64 to 192 waves are 1-3% slower on large lists and
+// the same on small ones, 384 and 512 no faster.  With a completion signal
+// every wave releases its stores, so there 64 waves (kGatherShape) stand:
+// submit_direct of 1024 x 4 KiB into scattered pages 91 us against 100.
+constexpr int kSgUnits = 1024;
+constexpr ShapeDefaults kSgShape{kBytesPerWave, kMaxWaves, kMaxWaves, kDefaultUnroll, "GFD_ZC_WAVES", "GFD_ZC_UNROLL"};
+
+// slice: the table is the caller's list as it is.  Without it, each record is
+// one wave's work (the caller has cut the list into pieces already).
 int launch_gather_sg(const gfd_sg_entry* entries, int count, void* stream, GridDone done, bool slice = true) {
     if (count < 0 || (count > 0 && !entries)) return (int)hipErrorInvalidValue;
     if (count == 0) return 0;
-    // Sizes are in the entry table, not known here: shape for 4 KiB entries.
-    const int target = short_list_waves();
-    const uint32_t pieces = slice && 2 * count <= target ? (uint32_t)(target / count) : 1u;
-    const Shape s = shape_for((uint64_t)count * pieces, (uint64_t)count * pieces * 4096);
+    const uint32_t pieces = slice && 2 * (int64_t)count <= kSgUnits ? (uint32_t)(kSgUnits / count) : 1u;
+    const Shape s = shape_for((uint64_t)count * pieces, (uint64_t)count * pieces * 4096,
+                              done.host_word ? kGatherShape : kSgShape);
     if (s.lds)
         hipLaunchKernelGGL(zc_gather_sg<true>, dim3(s.blocks), dim3(kBlock), 0, (hipStream_t)stream, entries,
                            (uint32_t)count, pieces, s.per_wave, s.unroll, done);

@@ -156,3 +156,38 @@ def test_tiles_any_alignment(size, skew, helpers):
     got = dst.download()
     assert (got[ds:ds + n * size] == host.array[ss:ss + n * size]).all()
     assert (got[:ds] == GUARD).all() and (got[ds + n * size:] == GUARD).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("count", [1, 2, 3, 63, 64, 65, 255, 511, 512, 513, 1025])
+@pytest.mark.parametrize("signal", [False, True])
+def test_entry_list_slices(count, signal):
+    """Lists of at most 512 entries are cut into 1024 / count slices each, taken
+    by the waves in strides; longer ones whole.  Sizes from 0 bytes (an empty
+    entry) to some KiB, so that slices are empty, whole and partial."""
+    print("slices count=%d signal=%d" % (count, signal), flush=True)
+    rng = np.random.default_rng(count)
+    size = rng.choice([0, 1, 16, 100, 1000, 16384, 30001], count).astype(np.uint64)
+    size[0] = 5000
+    start = np.concatenate([[0], np.cumsum(size + np.uint64(7))[:-1]]).astype(np.uint64)
+    total = int(start[-1] + size[-1]) + 64
+    host, dev = gfd_amd.HostBuffer(total), gfd_amd.DeviceBuffer(total)
+    host.array[:] = rng.integers(0, 256, total, dtype=np.uint8)
+    dev.fill(GUARD)
+    want = np.full(total, GUARD, np.uint8)
+    for o, n in zip(start.astype(int), size.astype(int)):
+        want[o:o + n] = host.array[o:o + n]
+    table = np.stack([np.uint64(dev.ptr) + start, np.uint64(host.ptr) + start, size], 1)
+    t = gfd_amd.DeviceBuffer(table.nbytes)
+    t.upload(table)
+    if signal:
+        word, counter = gfd_amd.HostBuffer(64, gfd_amd.HOST_COHERENT), gfd_amd.DeviceBuffer(64)
+        counter.fill(0)
+        word.array[:] = 0
+        assert gfd_amd.lib().gfd_zero_copy_gather_signal(t.ptr, count, counter.ptr, word.ptr, 77, None) == 0
+        gfd_amd.synchronize()
+        assert int(word.array.view(np.uint64)[0]) == 77 and (counter.download()[:4] == 0).all()
+    else:
+        gfd_amd.zero_copy_gather(t.ptr, count)
+        gfd_amd.synchronize()
+    assert (dev.download() == want).all()
