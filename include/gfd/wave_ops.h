@@ -313,7 +313,14 @@ __device__ __forceinline__ uint64_t copy_batch(int u, uint64_t md, uint64_t ms, 
 
 // Make this wave's global stores visible device-wide before a flag is raised
 // (producer side) / see other waves' stores after a flag is seen (consumer).
-__device__ __forceinline__ void release_agent() { __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent"); }
+// The release writes the XCD's L2 back (buffer_wbl2), which is done when
+// vmcnt is 0 again.  The compiler leaves that wait out where it sees no other
+// memory operation pending (after an explicit s_waitcnt, say), so it is
+// written here: 0x0F70 waits for vmcnt(0) alone.
+__device__ __forceinline__ void release_agent() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+    __builtin_amdgcn_s_waitcnt(0x0F70);
+}
 __device__ __forceinline__ void acquire_agent() { __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent"); }
 
 __device__ __forceinline__ int lds_load(const int* p) {
