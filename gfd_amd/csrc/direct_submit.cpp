@@ -88,6 +88,14 @@ int zc_fill_sg_table(const SGEntry* in, int count, size_t total, SGEntry* out, i
     return count;
 }
 
+// Pieces the zero-copy kernel's list is cut into: its short-list waves, or
+// twice as many where the entries alone take up more than a third of them (the
+// pieces would be large, and the waves unequal).  Measured on MI355X, 64
+// against 128: 40 entries of up to 20 KB 22.8 -> 21.8 us, 60 of up to 30 KB
+// 32.0 -> 30.2, 40 of up to 100 KB 56.1 -> 53.5; but 20 of up to 40 KB 21.0
+// -> 21.6.
+static int cut_waves(int count, int waves) { return 3 * (int64_t)count > waves ? 2 * waves : waves; }
+
 void run_copy_chunk(void* p, int chunk, size_t off, size_t len) {
     RunCopyCtx* c = (RunCopyCtx*)p;
     const size_t end = off + len;
@@ -256,7 +264,7 @@ int CpuPollingThread::direct_zero_copy(const SGEntry* entries, int count, size_t
         }
         bool cut = false;
         static const int kWaves = gfd_zero_copy_target_waves();
-        const int n = zc_fill_sg_table(entries, count, total, zc_table_, zc_table_cap_, &cut, kWaves);
+        const int n = zc_fill_sg_table(entries, count, total, zc_table_, zc_table_cap_, &cut, cut_waves(count, kWaves));
         rc = (cut ? gfd_zero_copy_gather_signal_presliced : gfd_zero_copy_gather_signal)(
             reinterpret_cast<const gfd_sg_entry*>(zc_table_), n, zc_counter_, zc_done_, gen, zc_stream_);
     }
@@ -321,7 +329,7 @@ int CpuPollingThread::zc_launch_head(const SGEntry* entries, int k, bool uniform
         for (int i = 0; i < k; i++) bytes += entries[i].size;
         bool cut = false;
         static const int kWaves = gfd_zero_copy_target_waves();
-        const int n = zc_fill_sg_table(entries, k, bytes, zc_table_, zc_table_cap_, &cut, kWaves);
+        const int n = zc_fill_sg_table(entries, k, bytes, zc_table_, zc_table_cap_, &cut, cut_waves(k, kWaves));
         rc = (cut ? gfd_zero_copy_gather_signal_presliced : gfd_zero_copy_gather_signal)(
             reinterpret_cast<const gfd_sg_entry*>(zc_table_), n, zc_counter_, zc_done_, g, zc_stream_);
     }

@@ -96,7 +96,7 @@ __global__ __launch_bounds__(kBlock) void zc_gather_tokens(const uint64_t* __res
         }
         gfd::wave::copy_batch(unroll, md, ms, mn, nb, &lds[wid], kLds ? stage[wid] : nullptr);
     }
-    gfd::wave::signal_grid_done(done, gridDim.x * kWavesPerBlock);
+    gfd::wave::signal_grid_done(done);
 }
 
 // Reverse direction (KV-page offload): token j of num_tokens is read from HBM
@@ -127,7 +127,7 @@ __global__ __launch_bounds__(kBlock) void zc_scatter_tokens(const uint64_t* __re
         }
         gfd::wave::copy_batch(unroll, md, ms, mn, nb, &lds[wid], kLds ? stage[wid] : nullptr);
     }
-    gfd::wave::signal_grid_done(done, gridDim.x * kWavesPerBlock);
+    gfd::wave::signal_grid_done(done);
 }
 
 // Generic SG list: any sizes, any (disjoint) destinations, same batching.
@@ -165,7 +165,7 @@ __global__ __launch_bounds__(kBlock) void zc_gather_sg(const gfd_sg_entry* __res
         }
         gfd::wave::copy_batch(unroll, md, ms, mn, nb, &lds[wid], kLds ? stage[wid] : nullptr);
     }
-    gfd::wave::signal_grid_done(done, gridDim.x * kWavesPerBlock);
+    gfd::wave::signal_grid_done(done);
 }
 
 int env_int(const char* name, int dflt) {
@@ -278,19 +278,20 @@ int short_list_waves() { return std::max(4, env_int(kGatherShape.waves_env, kGat
 // alone.  512 units leave 3% more at 64 entries, 2048 and 4096 cost 5-15% on
 // a single 1 MiB entry; 64 to 192 waves are 1-3% slower on large lists and
 // the same on small ones, 384 and 512 no faster.  With a completion signal
-// every wave releases its stores, so there 64 waves (kGatherShape) stand:
-// submit_direct of 1024 x 4 KiB into scattered pages 91 us against 100.
+// every workgroup writes its L2 back, so there 64 waves (kGatherShape) stand:
+// submit_direct of 1024 x 4 KiB into scattered pages 89 us against 92.
 constexpr int kSgUnits = 1024;
 constexpr ShapeDefaults kSgShape{kBytesPerWave, kMaxWaves, kMaxWaves, kDefaultUnroll, "GFD_ZC_WAVES", "GFD_ZC_UNROLL"};
 
 // slice: the table is the caller's list as it is.  Without it, each record is
-// one wave's work (the caller has cut the list into pieces already).
+// one wave's work (the caller has cut the list into pieces already), up to
+// kMaxWaves of them.
 int launch_gather_sg(const gfd_sg_entry* entries, int count, void* stream, GridDone done, bool slice = true) {
     if (count < 0 || (count > 0 && !entries)) return (int)hipErrorInvalidValue;
     if (count == 0) return 0;
     const uint32_t pieces = slice && 2 * (int64_t)count <= kSgUnits ? (uint32_t)(kSgUnits / count) : 1u;
     const Shape s = shape_for((uint64_t)count * pieces, (uint64_t)count * pieces * 4096,
-                              done.host_word ? kGatherShape : kSgShape);
+                              done.host_word && slice ? kGatherShape : kSgShape);
     if (s.lds)
         hipLaunchKernelGGL(zc_gather_sg<true>, dim3(s.blocks), dim3(kBlock), 0, (hipStream_t)stream, entries,
                            (uint32_t)count, pieces, s.per_wave, s.unroll, done);
