@@ -6,7 +6,7 @@
 // builds the lists on the GPU).  Here the whole path stays on the GPU:
 //
 //   1. moe_top2_kernel   — top-2 experts per token from the logits (ties go to
-//                          the lower expert id), one wave64 per token.
+//                          the lower expert id), 16 lanes per token.
 //   2. moe_lists_kernel  — one workgroup per expert builds its row list in token
 //                          order (stable; no atomics), plus the expert offsets.
 //                          Rows are packed expert-major.
@@ -43,76 +43,184 @@ constexpr uint64_t kSpinLimit = 1ull << 26;  // LDS flag polls before giving up
 
 // ---------------------------------------------------------------- routing
 
-__device__ __forceinline__ void wave_argmax(float& v, int& idx) {
+// A token's experts are shared by 16 lanes, four each (lane l: experts l, l +
+// 16, l + 32, l + 48, -inf where there is none).
+constexpr int kTokLanes = 16, kTokExperts = 64 / kTokLanes;
+
+// Reductions over a token's lanes, one DPP row, in every lane: l with 15 - l,
+// with 7 - l in each half, then l ^ 2 and l ^ 1.  Each step is one
+// instruction; as LDS permutes, or carrying (value, expert) pairs through
+// compares and selects, they bound a workgroup of 16 waves.
+template <int kCtrl>
+__device__ __forceinline__ int dpp(int v) { return __builtin_amdgcn_mov_dpp(v, kCtrl, 0xF, 0xF, true); }
+__device__ __forceinline__ float row_max(float v) {
+    v = fmaxf(v, __int_as_float(dpp<0x140>(__float_as_int(v))));
+    v = fmaxf(v, __int_as_float(dpp<0x141>(__float_as_int(v))));
+    v = fmaxf(v, __int_as_float(dpp<0x4E>(__float_as_int(v))));
+    return fmaxf(v, __int_as_float(dpp<0xB1>(__float_as_int(v))));
+}
+__device__ __forceinline__ int row_min(int v) {
+    v = min(v, dpp<0x140>(v));
+    v = min(v, dpp<0x141>(v));
+    v = min(v, dpp<0x4E>(v));
+    return min(v, dpp<0xB1>(v));
+}
+
+// The lowest expert that holds the largest of the token's logits, in every
+// lane.  A NaN is never the largest; 0 if all are NaN.
+__device__ __forceinline__ int argmax16(const float (&x)[kTokExperts], int num_experts, int lane) {
+    const float top = row_max(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])));
+    int i = 64;
 #pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-        const float ov = __shfl_xor(v, off, kWave);
-        const int oi = __shfl_xor(idx, off, kWave);
-        if (ov > v || (ov == v && oi < idx)) {
-            v = ov;
-            idx = oi;
-        }
+    for (int k = kTokExperts - 1; k >= 0; k--) i = x[k] == top ? lane + k * kTokLanes : i;
+    i = row_min(i);
+    return i < num_experts ? i : 0;
+}
+
+typedef int int2v __attribute__((ext_vector_type(2), aligned(4)));
+
+// The lane's logits of token min(t, num_tokens - 1), one token per 16 lanes.
+__device__ __forceinline__ void load_logits(float (&x)[kTokExperts], const float* __restrict__ logits, int t,
+                                            int num_tokens, int num_experts, int lane) {
+    const float* row = logits + (size_t)min(t, num_tokens - 1) * num_experts;
+#pragma unroll
+    for (int k = 0; k < kTokExperts; k++) {
+        // Past the last expert: a valid load whose value is not kept.
+        const int e = lane + k * kTokLanes;
+        const float v = row[min(e, num_experts - 1)];
+        x[k] = e < num_experts ? v : -INFINITY;
     }
 }
 
-__global__ __launch_bounds__(256) void moe_top2_kernel(const float* __restrict__ logits, int num_tokens,
-                                                       int num_experts, int* __restrict__ top2) {
-    const int t = (int)((blockIdx.x * blockDim.x + threadIdx.x) / kWave);
-    const int lane = (int)(threadIdx.x % kWave);
-    if (t >= num_tokens) return;  // uniform per wave
-    const float x = lane < num_experts ? logits[(size_t)t * num_experts + lane] : -INFINITY;
-    float v = x;
-    int i = lane;
-    wave_argmax(v, i);
-    const int first = i;
-    v = (lane == first || lane >= num_experts) ? -INFINITY : x;
-    i = lane;
-    wave_argmax(v, i);
-    if (lane == 0) {
-        top2[2 * t] = first;
-        top2[2 * t + 1] = i;
-    }
+// The token's two experts, in all of its lanes.
+__device__ __forceinline__ int2v top2_of(float (&x)[kTokExperts], int num_experts, int lane) {
+    const int first = argmax16(x, num_experts, lane);
+#pragma unroll
+    for (int k = 0; k < kTokExperts; k++)
+        if (lane + k * kTokLanes == first) x[k] = -INFINITY;
+    return int2v{first, argmax16(x, num_experts, lane)};
+}
+
+// Latency bound: 4 loads, then two chains of 8 cross-lane steps.  16 tokens
+// per workgroup, so that 4096 tokens reach every CU (2.4 us; 3.8 with a wave
+// and 24 LDS permutes per token); 2 or 4 tokens per 16 lanes were slower from
+// 10000 tokens on.
+constexpr int kTop2Block = 256, kTokBlock = kTop2Block / kTokLanes;
+__global__ __launch_bounds__(kTop2Block) void moe_top2_kernel(const float* __restrict__ logits, int num_tokens,
+                                                              int num_experts, int* __restrict__ top2) {
+    const int lane = (int)(threadIdx.x % kTokLanes);
+    const int t = (int)(blockIdx.x * kTokBlock + threadIdx.x / kTokLanes);
+    float x[kTokExperts];
+    load_logits(x, logits, t, num_tokens, num_experts, lane);
+    const int2v p = top2_of(x, num_experts, lane);
+    if (lane == 0 && t < num_tokens) *reinterpret_cast<int2v*>(top2 + 2 * (size_t)t) = p;
 }
 
 // Workgroup e: offsets[e] = number of (token, choice) pairs routed to experts
 // below e; row_token[offsets[e] + k] = k-th token (in token order) routed to e.
-__global__ __launch_bounds__(256) void moe_lists_kernel(const int* __restrict__ top2, int num_tokens,
-                                                        int num_experts, int* __restrict__ offsets,
-                                                        int* __restrict__ row_token) {
-    __shared__ int wave_sum[4];
-    __shared__ int block_base;
+// pair(t) gives token t's two experts.  The workgroup's 16 waves own one run
+// of tokens each.  Pass 1 counts the run's hits and the pairs below e, U reads
+// in flight per lane; one exchange of the waves' counts gives every wave its
+// first slot; pass 2 places the run's hits by ballots.  Runs of at most 64 U
+// tokens (1024 U in all) stay in registers between the passes.  Bound by the
+// latency of the reads: at 4096 x 64 a kernel that walked all pairs twice with
+// 4 waves, one read in flight and two barriers per 256 tokens took 14.0 us,
+// this one 4.4; the whole routing 16.6 -> 9.2 us a call, at 20000 x 64 66 ->
+// 12.3, at 65536 x 64 204 -> 29.
+constexpr int kListWaves = 16;
+template <int U, typename Pair>
+__device__ __forceinline__ void place_rows(Pair pair, int num_tokens, int num_experts, int* __restrict__ offsets,
+                                           int* __restrict__ row_token) {
+    __shared__ int wave_hits[kListWaves], wave_below[kListWaves];
     const int e = (int)blockIdx.x;
-    const int tid = (int)threadIdx.x;
-    const int lane = tid % kWave, wave = tid / kWave;
-
-    // Offset of this expert: pairs routed to lower experts.
-    int below = 0;
-    for (int t = tid; t < num_tokens; t += 256) below += (top2[2 * t] < e) + (top2[2 * t + 1] < e);
-    for (int off = 32; off >= 1; off >>= 1) below += __shfl_xor(below, off, kWave);
-    if (lane == 0) wave_sum[wave] = below;
+    const int lane = (int)(threadIdx.x % kWave), wave = (int)(threadIdx.x / kWave);
+    // Runs are whole groups of 64 tokens.
+    const int groups = (num_tokens + kWave - 1) / kWave;
+    const int per = (groups + kListWaves - 1) / kListWaves;
+    const int g0 = min(wave * per, groups), g1 = min(g0 + per, groups);
+    int2v p[U];
+    auto read = [&](int g) {
+#pragma unroll
+        for (int k = 0; k < U; k++) {
+            const int t = (g + k) * kWave + lane;
+            const int2v v = pair(min(t, num_tokens - 1));
+            p[k] = g + k < g1 && t < num_tokens ? v : int2v{-1, -1};
+        }
+    };
+    int hits = 0, below = 0;
+    for (int g = g0; g < g1; g += U) {
+        read(g);
+#pragma unroll
+        for (int k = 0; k < U; k++) {
+            hits += __popcll(__ballot(p[k].x == e || p[k].y == e));
+            below += __popcll(__ballot((uint32_t)p[k].x < (uint32_t)e)) +
+                     __popcll(__ballot((uint32_t)p[k].y < (uint32_t)e));
+        }
+    }
+    if (lane == 0) {
+        wave_hits[wave] = hits;
+        wave_below[wave] = below;
+    }
     __syncthreads();
-    if (tid == 0) {
-        block_base = wave_sum[0] + wave_sum[1] + wave_sum[2] + wave_sum[3];
-        offsets[e] = block_base;
+    int at = 0;
+#pragma unroll
+    for (int w = 0; w < kListWaves; w++) at += wave_below[w] + (w < wave ? wave_hits[w] : 0);
+    if (threadIdx.x == 0) {
+        offsets[e] = at;
         if (e == num_experts - 1) offsets[num_experts] = 2 * num_tokens;
     }
-    __syncthreads();
-
-    // Stable placement: block-wide exclusive prefix over token order.
-    int running = block_base;
-    for (int base = 0; base < num_tokens; base += 256) {
-        const int t = base + tid;
-        const bool hit = t < num_tokens && (top2[2 * t] == e || top2[2 * t + 1] == e);
-        const uint64_t mask = __ballot(hit);
-        const int before_in_wave = __popcll(mask & ((1ull << lane) - 1ull));
-        __syncthreads();
-        if (lane == 0) wave_sum[wave] = __popcll(mask);
-        __syncthreads();
-        int before_waves = 0;
-        for (int w = 0; w < wave; w++) before_waves += wave_sum[w];
-        if (hit) row_token[running + before_waves + before_in_wave] = t;
-        running += wave_sum[0] + wave_sum[1] + wave_sum[2] + wave_sum[3];
+    const uint64_t lower = (1ull << lane) - 1ull;
+    for (int g = g0; g < g1; g += U) {
+        if (per > U) read(g);
+#pragma unroll
+        for (int k = 0; k < U; k++) {
+            const bool hit = p[k].x == e || p[k].y == e;
+            const uint64_t mask = __ballot(hit);
+            if (hit) row_token[at + __popcll(mask & lower)] = (g + k) * kWave + lane;
+            at += __popcll(mask);
+        }
     }
+}
+
+__global__ __launch_bounds__(kListWaves * 64) void moe_lists_kernel(const int* __restrict__ top2, int num_tokens,
+                                                                   int num_experts, int* __restrict__ offsets,
+                                                                   int* __restrict__ row_token) {
+    place_rows<8>([=](int t) { return *reinterpret_cast<const int2v*>(top2 + 2 * (size_t)t); }, num_tokens,
+                  num_experts, offsets, row_token);
+}
+
+// Both steps in one launch for few tokens: every expert's workgroup works the
+// pairs of all tokens out again, into LDS, and writes its share of top2.  The
+// work repeated costs 0.6 us per 64 tokens and the launch saved 4.3 us, so up
+// to 512 tokens: 60 x 4 9.6 -> 6.8 us a call, 256 x 64 9.3 -> 6.6, 512 x 64
+// 9.3 -> 7.5 (1000 x 16 would be 12.2 against 9.0).
+constexpr int kFusedTokens = 512;
+__global__ __launch_bounds__(kListWaves * 64) void moe_route_kernel(const float* __restrict__ logits, int num_tokens,
+                                                                   int num_experts, int* __restrict__ top2,
+                                                                   int* __restrict__ offsets,
+                                                                   int* __restrict__ row_token) {
+    __shared__ int2v pairs[kFusedTokens];
+    constexpr int kGroups = kListWaves * kWave / kTokLanes;  // tokens at a time
+    constexpr int kAhead = 4;                                // of each group's, loaded together
+    const int lane = (int)(threadIdx.x % kTokLanes), group = (int)(threadIdx.x / kTokLanes);
+    for (int t0 = group; t0 < num_tokens; t0 += kAhead * kGroups) {
+        float x[kAhead][kTokExperts];
+#pragma unroll
+        for (int a = 0; a < kAhead; a++) load_logits(x[a], logits, t0 + a * kGroups, num_tokens, num_experts, lane);
+#pragma unroll
+        for (int a = 0; a < kAhead; a++) {
+            if (__builtin_amdgcn_readfirstlane(t0 + a * kGroups) >= num_tokens) break;  // none for the whole wave
+            const int2v p = top2_of(x[a], num_experts, lane);
+            if (lane == 0 && t0 + a * kGroups < num_tokens) pairs[t0 + a * kGroups] = p;
+        }
+    }
+    __syncthreads();
+    const int share = (num_tokens + (int)gridDim.x - 1) / (int)gridDim.x;
+    const int s0 = (int)blockIdx.x * share, s1 = min(s0 + share, num_tokens);
+    for (int t = s0 + (int)threadIdx.x; t < s1; t += kListWaves * kWave)
+        *reinterpret_cast<int2v*>(top2 + 2 * (size_t)t) = pairs[t];
+    place_rows<1>([&](int t) { return pairs[t]; }, num_tokens, num_experts, offsets,
+                                                    row_token);
 }
 
 // ------------------------------------------------------ gather + RMSNorm
@@ -296,11 +404,15 @@ int moe_scratch_ptr(int** out) {
 
 int launch_route(const float* logits, int num_tokens, int num_experts, int* top2, int* offsets, int* row_token,
                  hipStream_t st) {
-    const int waves_per_block = 256 / kWave;
-    hipLaunchKernelGGL(moe_top2_kernel, dim3((num_tokens + waves_per_block - 1) / waves_per_block), dim3(256), 0, st,
+    if (num_tokens <= kFusedTokens) {
+        hipLaunchKernelGGL(moe_route_kernel, dim3(num_experts), dim3(kListWaves * kWave), 0, st, logits, num_tokens,
+                           num_experts, top2, offsets, row_token);
+        return (int)hipGetLastError();
+    }
+    hipLaunchKernelGGL(moe_top2_kernel, dim3((num_tokens + kTokBlock - 1) / kTokBlock), dim3(kTop2Block), 0, st,
                        logits, num_tokens, num_experts, top2);
-    hipLaunchKernelGGL(moe_lists_kernel, dim3(num_experts), dim3(256), 0, st, top2, num_tokens, num_experts, offsets,
-                       row_token);
+    hipLaunchKernelGGL(moe_lists_kernel, dim3(num_experts), dim3(kListWaves * kWave), 0, st, top2, num_tokens,
+                       num_experts, offsets, row_token);
     return (int)hipGetLastError();
 }
 

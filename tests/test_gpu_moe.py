@@ -122,3 +122,55 @@ def test_gather_flags_out_of_range_token():
                               None, 1e-6, 4, m.d_err.ptr)
     gfd_amd.synchronize()
     assert int(m.d_err.download().view(np.int32)[0]) & 4
+
+
+# Tokens around the one-launch limit (512), the waves' groups (64) and the
+# runs kept in registers (8192); experts around the 16 lanes of a token.
+@pytest.mark.parametrize("T", [1, 15, 64, 65, 511, 512, 513, 1025, 8191, 8192, 8193, 20001])
+@pytest.mark.parametrize("E", [2, 3, 16, 17, 63, 64])
+def test_route_edges(T, E):
+    """top2, offsets and row lists exact, with ties (lower expert first), -inf
+    logits, and guards behind every output."""
+    print("route T=%d E=%d" % (T, E), flush=True)
+    rng = np.random.default_rng(T * 100 + E)
+    logits = rng.integers(-3, 4, (T, E)).astype(np.float32)  # many ties
+    logits[rng.random((T, E)) < 0.2] = -np.inf
+    logits[:, rng.permutation(E)[:2]] = (4.0, 5.0)  # two finite ones in every row
+    logits[: T // 2] += rng.standard_normal((T // 2, E), dtype=np.float32)
+    top2 = oracle.moe_top2(logits)
+    offsets, rows = oracle.moe_lists(top2, E)
+    d = gfd_amd.DeviceBuffer(logits.nbytes)
+    d.upload(logits)
+    outs = [gfd_amd.DeviceBuffer(4 * n + 64) for n in (2 * T, E + 1, 2 * T)]
+    for o in outs:
+        o.fill(0xCD)
+    gfd_amd.moe_route(d.ptr, T, E, outs[0].ptr, outs[1].ptr, outs[2].ptr)
+    gfd_amd.synchronize()
+    got = [o.download() for o in outs]
+    for g, n in zip(got, (2 * T, E + 1, 2 * T)):
+        assert (g[4 * n:] == 0xCD).all()
+    assert (got[0][:8 * T].view(np.int32) == top2.reshape(-1)).all()
+    assert (got[1][:4 * (E + 1)].view(np.int32) == offsets).all()
+    k = len(rows)
+    assert (got[2][:4 * k].view(np.int32) == rows).all()
+
+
+@pytest.mark.parametrize("T", [300, 5000])
+def test_route_of_nan_rows_stays_in_range(T):
+    """A row that holds NaN still routes to experts that exist."""
+    E = 5
+    logits = np.random.default_rng(T).standard_normal((T, E), dtype=np.float32)
+    logits[np.random.default_rng(T + 1).random((T, E)) < 0.4] = np.nan
+    d, t2, off, rows = [gfd_amd.DeviceBuffer(n) for n in (logits.nbytes, 8 * T, 4 * (E + 1), 8 * T)]
+    d.upload(logits)
+    rows.fill(0)
+    gfd_amd.moe_route(d.ptr, T, E, t2.ptr, off.ptr, rows.ptr)
+    gfd_amd.synchronize()
+    top2 = t2.download().view(np.int32)
+    assert (top2 >= 0).all() and (top2 < E).all()
+    clean = ~np.isnan(logits).any(1)
+    assert (top2.reshape(T, 2)[clean] == oracle.moe_top2(logits[clean])).all()
+    o = off.download().view(np.int32)
+    assert o[0] == 0 and o[E] == 2 * T and (np.diff(o) >= 0).all()
+    r = rows.download().view(np.int32)
+    assert (r >= 0).all() and (r < T).all()
