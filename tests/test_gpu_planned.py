@@ -93,6 +93,40 @@ def test_plan_expert_entries_stable_order(total, experts):
         assert (got["dst"] == np.uint64(1 << 44) + np.arange(n, dtype=np.uint64) * np.uint64(t)).all()
 
 
+# Edges of a wave's run (64, 512), a workgroup's range (1024, 8192) and the
+# workgroups (8 x 1024, 8 x 8192), and runs longer than one round of reads.
+@pytest.mark.parametrize("total", [0, 63, 64, 65, 1023, 1024, 2049, 8191, 8192, 8193, 65536, 65537, 140001])
+@pytest.mark.parametrize("where", ["device", "host"])
+def test_plan_expert_entries_edges(total, where):
+    log("plan edges total=%d table in %s memory" % (total, where))
+    rng = np.random.default_rng(total)
+    routing = rng.integers(0, 3, total).astype(np.int32)
+    routing[total // 2:] = rng.integers(0, 40, total - total // 2)
+    # the table at an address that is 4 but not 16 bytes aligned
+    if where == "device":
+        tab = gfd_amd.DeviceBuffer(total * 4 + 16)
+        if total:
+            tab.upload(routing, offset=4)
+    else:
+        tab = gfd_amd.HostBuffer(total * 4 + 16)
+        tab.array[4:4 + total * 4] = routing.view(np.uint8)
+    for e in (0, 2, 39):
+        toks = np.nonzero(routing == e)[0]
+        entries = gfd_amd.HostBuffer((len(toks) + 1) * ENTRY_DTYPE.itemsize)
+        entries.array[:] = 0xCD
+        count = gfd_amd.HostBuffer(64)
+        count.array.view(np.int32)[0] = -1
+        gfd_amd.plan_expert_entries(tab.ptr + 4, total, e, 1 << 40, 192, 1 << 44, 64, entries.ptr, count.ptr)
+        gfd_amd.synchronize()
+        n = int(count.array.view(np.int32)[0])
+        assert n == len(toks)
+        got = entries.array.view(ENTRY_DTYPE)[:n]
+        assert (got["src"] == np.uint64(1 << 40) + toks.astype(np.uint64) * np.uint64(192)).all()
+        assert (got["dst"] == np.uint64(1 << 44) + np.arange(n, dtype=np.uint64) * np.uint64(64)).all()
+        assert (got["size"] == 64).all()
+        assert (entries.array[n * ENTRY_DTYPE.itemsize:] == 0xCD).all()
+
+
 def test_plan_expert_entries_rejects_bad_args():
     buf = gfd_amd.DeviceBuffer(64)
     with pytest.raises(gfd_amd.GfdError):
