@@ -392,7 +392,8 @@ int warp_spec_run(const void* cpu_src, void* gpu_dst, uint32_t total_tokens, uin
     if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess)
         return fail(hipErrorOutOfMemory, "gfd_warp_spec_run: event creation failed");
     int rc = 0;
-    const auto p = s.get_launch_params();
+    auto p = s.get_launch_params();
+    if (consumer == kWsRmsSin) p.grid = s.split_grid();  // a kSplitsChunks functor, as in launch()
     for (int it = 0; it < iters && rc == 0; it++) {
         // launch() with the HIP events around the kernel alone: before_launch
         // clears the signals with a blocking memset first.
@@ -433,6 +434,7 @@ int warp_spec_run(const void* cpu_src, void* gpu_dst, uint32_t total_tokens, uin
         else if (!ok) rc = fail(hipErrorLaunchFailure, "gfd_warp_spec_run: kernel reported an error or missing tiles");
     }
     fill_ws_result(s, c, res);
+    res->grid = (int)p.grid;
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     return rc;

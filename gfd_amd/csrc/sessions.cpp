@@ -128,6 +128,14 @@ WarpSpecSession::LaunchParams WarpSpecSession::get_launch_params() const {
     return p;
 }
 
+unsigned WarpSpecSession::split_grid() const {
+    const unsigned tiles = config_.total_tiles(), chunks = config_.chunks_per_tile();
+    unsigned parts = 1;
+    if (config_.num_blocks <= 0 && tiles > 0 && tiles <= (unsigned)MAX_TILES)
+        while (chunks % (2 * parts) == 0 && tiles * 2 * parts <= kSplitGrid) parts *= 2;
+    return parts > 1 ? tiles * parts : (unsigned)num_blocks_;
+}
+
 void WarpSpecSession::reset() {
     if (running_) synchronize();
     if (!tq_) return;

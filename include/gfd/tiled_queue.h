@@ -39,4 +39,19 @@ struct TileDeviceCounters {
 constexpr int TILE_DEVICE_COUNTER_WORDS = (int)(sizeof(TileDeviceCounters) / sizeof(uint64_t));
 static_assert(sizeof(TileDeviceCounters) == 64, "TileDeviceCounters is one cache line");
 
+namespace warp_spec {
+
+// A compute functor that declares `static constexpr bool kSplitsChunks = true`
+// (see warp_spec.h).
+template <typename F, typename = void>
+struct _splits_chunks {
+    static constexpr bool value = false;
+};
+template <typename F>
+struct _splits_chunks<F, decltype((void)F::kSplitsChunks)> {
+    static constexpr bool value = F::kSplitsChunks;
+};
+
+}  // namespace warp_spec
+
 }  // namespace gfd

@@ -104,14 +104,21 @@ struct _TileSlot {
 // ends.  The functor sees each group as a ChunkView of that group's tokens.
 // Functors without the declaration see each chunk once, on its own wave, as
 // with the reference.
-template <typename F, typename = void>
-struct _splits_chunks {
-    static constexpr bool value = false;
-};
-template <typename F>
-struct _splits_chunks<F, decltype((void)F::kSplitsChunks)> {
-    static constexpr bool value = F::kSplitsChunks;
-};
+// (The trait _splits_chunks is in tiled_queue.h: the session reads it too.)
+//
+// A launch of such a functor on more workgroups than tiles cuts every tile
+// into parts of whole chunks, and each part is a workgroup's work like a tile
+// of its own: part u of S per tile is tokens [u * T / S, (u + 1) * T / S).
+// One workgroup moves at most ~13 GB/s over PCIe and computes the last chunk
+// with its own waves only, so a launch of few tiles left the link and the chip
+// idle: 256 tokens of 4 KiB (2 tiles of 4 chunks) took 102 us in 2 workgroups and
+// take 47 in 8.
+__device__ __forceinline__ uint32_t _tile_parts(uint32_t total_tiles, uint32_t chunks) {
+    uint32_t parts = 1;
+    if (total_tiles <= (uint32_t)MAX_TILES)  // every tile has a progress word, which counts its parts
+        while (chunks % (2 * parts) == 0 && (uint64_t)total_tiles * 2 * parts <= gridDim.x) parts *= 2;
+    return parts;
+}
 
 // Wait until chunk k of the slot's tile at `epoch` has landed while some of
 // its tokens are still unclaimed: 1 (landed, after an acquire), 0 (nothing
@@ -130,14 +137,14 @@ __device__ __forceinline__ int _wait_claimable(_TileSlot& sl, int epoch, uint32_
     return -1;
 }
 
-// Claim and compute token groups (G tokens) of chunk k of `tile`, the tile of
-// slot `sl` at epoch `epoch` (its seq), until none is left.  The chunk must
+// Claim and compute token groups (G tokens) of chunk k of `tile`, the tile (or
+// part of one, S to a tile, K chunks and T tokens each) of slot `sl` at epoch `epoch` (its seq), until none is left.  The chunk must
 // have landed (the caller saw chunk_done[k] == P and made an acquire).  The
 // group that completes the chunk counts it in `done`.
 template <typename ComputeFn>
-__device__ __forceinline__ void _compute_groups(_TileSlot& sl, int epoch, uint32_t tile, uint32_t k, uint32_t T,
-                                                uint32_t C, uint32_t G, uint32_t token_size, void* gpu_buffer,
-                                                ComputeFn& compute_fn) {
+__device__ __forceinline__ void _compute_groups(_TileSlot& sl, int epoch, uint32_t tile, uint32_t k, uint32_t S,
+                                                uint32_t K, uint32_t T, uint32_t C, uint32_t G, uint32_t token_size,
+                                                void* gpu_buffer, ComputeFn& compute_fn) {
     const int lane = wave::lane_id();
     for (;;) {
         // The retry loop is wave-uniform and only the compare-and-swap is
@@ -160,8 +167,8 @@ __device__ __forceinline__ void _compute_groups(_TileSlot& sl, int epoch, uint32
         v.base_ptr = (char*)gpu_buffer + (uint64_t)v.global_token_offset * token_size;
         v.token_size = token_size;
         v.size = n;
-        v.tile_id = tile;
-        v.chunk_id = k;
+        v.tile_id = tile / S;
+        v.chunk_id = tile % S * K + k;
         v.lane_id = lane;
         compute_fn(v);
         if (lane == 0) {
@@ -231,9 +238,12 @@ __device__ __forceinline__ void _tile_loop(TiledQueue* tq, void* gpu_buffer, con
     const int w = wave::wave_id();
     const int lane = wave::lane_id();
     const uint32_t C = tq->scheduler.tokens_per_chunk;
-    const uint32_t K = tq->scheduler.chunks_per_tile;
-    const uint32_t T = tq->scheduler.tokens_per_tile;
+    const uint32_t tile_chunks = tq->scheduler.chunks_per_tile;
+    const uint32_t tile_tokens = tq->scheduler.tokens_per_tile;
     const uint32_t total_tiles = tq->scheduler.total_tiles;
+    // What a workgroup claims: a tile, or one of S parts of it.
+    const uint32_t S = _splits_chunks<ComputeFn>::value ? _tile_parts(total_tiles, tile_chunks) : 1u;
+    const uint32_t K = tile_chunks / S, T = tile_tokens / S, units = total_tiles * S;
     const uint32_t token_size = tq->scheduler.token_size;
     TileDeviceCounters* cnt = tile_counters(tq);
     if (threadIdx.x < NSLOTS) {
@@ -250,12 +260,12 @@ __device__ __forceinline__ void _tile_loop(TiledQueue* tq, void* gpu_buffer, con
 
     // Waves after the compute waves are transfer helpers.
     const int nwaves = (int)(blockDim.x / wave::kWidth);
-    const int first_helper = 1 + NSLOTS * (int)K;
+    const int first_helper = 1 + NSLOTS * (int)tile_chunks;
     const int helpers = nwaves > first_helper ? nwaves - first_helper : 0;
     const uint64_t chunk_bytes = (uint64_t)C * token_size;
     const uint32_t P = _pieces_per_chunk(K, 1u + (uint32_t)helpers, chunk_bytes);
     const uint64_t piece_bytes = ((chunk_bytes + P - 1) / P + 1023) & ~1023ull;
-    const uint32_t active = gridDim.x < total_tiles ? gridDim.x : total_tiles;
+    const uint32_t active = gridDim.x < units ? gridDim.x : units;
     const int unroll = wave::transfer_unroll(active * (1u + (uint32_t)helpers));
 
     if (w == 0) {
@@ -269,7 +279,7 @@ __device__ __forceinline__ void _tile_loop(TiledQueue* tq, void* gpu_buffer, con
             uint64_t tile = 0;
             if (lane == 0) tile = __hip_atomic_fetch_add(&cnt->next_tile, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             tile = wave::broadcast0(tile);
-            const bool last = tile >= total_tiles;
+            const bool last = tile >= units;
             if (lane == 0) {
                 const int epoch = (int)(n / NSLOTS) + 1;
                 slots[s].tile = last ? TILE_END : (uint32_t)tile;
@@ -313,9 +323,13 @@ __device__ __forceinline__ void _tile_loop(TiledQueue* tq, void* gpu_buffer, con
                 break;
             }
             if (lane == 0) {
-                if (tile < (uint64_t)MAX_TILES)
+                bool whole = true;  // the tile has landed
+                if (S > 1)
+                    whole = __hip_atomic_fetch_add(&tile_done_words(cnt)[tile / S], (uint64_t)T, __ATOMIC_RELEASE,
+                                                   __HIP_MEMORY_SCOPE_AGENT) + T == tile_tokens;
+                else if (tile < (uint64_t)MAX_TILES)
                     __hip_atomic_store(&tile_done_words(cnt)[tile], (uint64_t)T, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-                __hip_atomic_fetch_add(&cnt->tiles_done, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (whole) __hip_atomic_fetch_add(&cnt->tiles_done, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
         }
         if (lane == 0) wave::lds_store(&job.seq, -1);  // helpers exit
@@ -345,11 +359,11 @@ __device__ __forceinline__ void _tile_loop(TiledQueue* tq, void* gpu_buffer, con
             }
             want = seq + 1;
         }
-    } else if ((uint32_t)(w - 1) < NSLOTS * K && _splits_chunks<ComputeFn>::value) {
+    } else if ((uint32_t)(w - 1) < NSLOTS * tile_chunks && _splits_chunks<ComputeFn>::value) {
         // ---------------- compute waves sharing the chunks: slot g, chunk k first
-        const int g = (int)((uint32_t)(w - 1) / K);
+        const int g = (int)((uint32_t)(w - 1) / tile_chunks);
         const uint32_t k = (uint32_t)(w - 1) % K;
-        uint32_t G = C / (NSLOTS * K);
+        uint32_t G = C / (NSLOTS * tile_chunks);
         G = G ? G : 1u;
         for (int n = 1;; n++) {
             if (!wave::wait_lds_eq(&slots[g].seq, n)) {
@@ -369,7 +383,7 @@ __device__ __forceinline__ void _tile_loop(TiledQueue* tq, void* gpu_buffer, con
                         const uint32_t k2 = (k + i) % K;
                         const int r = _wait_claimable(other, epoch, k2, P, C);
                         if (r < 0) break;  // its own waves report a stall
-                        if (r > 0) _compute_groups(other, epoch, otile, k2, T, C, G, token_size, gpu_buffer, compute_fn);
+                        if (r > 0) _compute_groups(other, epoch, otile, k2, S, K, T, C, G, token_size, gpu_buffer, compute_fn);
                     }
                 }
                 break;
@@ -386,7 +400,7 @@ __device__ __forceinline__ void _tile_loop(TiledQueue* tq, void* gpu_buffer, con
                     if (lane == 0) __hip_atomic_fetch_or(&cnt->error, WS_ERR_CHUNK_WAIT, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                     ok = false;
                 } else if (r > 0) {
-                    _compute_groups(slots[g], n, tile, k2, T, C, G, token_size, gpu_buffer, compute_fn);
+                    _compute_groups(slots[g], n, tile, k2, S, K, T, C, G, token_size, gpu_buffer, compute_fn);
                 }
             }
             if (!ok) break;

@@ -50,7 +50,7 @@ struct WarpSpecConfig {
     // optional
     uint32_t tokens_per_tile = 128;
     uint32_t tokens_per_chunk = 0;  // 0 = automatic
-    int num_blocks = 0;             // 0 = one workgroup per tile, at most one per CU
+    int num_blocks = 0;             // 0 = one workgroup per tile, at most one per CU (more for few tiles: split_grid())
     int numa_node = 0;              // kept for API compatibility
     bool use_copy_engine = true;    // kept for API compatibility (data moves zero-copy)
     bool double_buffer = false;
@@ -116,6 +116,16 @@ public:
         unsigned block;
     };
     LaunchParams get_launch_params() const;
+    // The grid launch() uses for a functor with kSplitsChunks: unless the
+    // configuration sets num_blocks, few tiles are cut into parts of whole
+    // chunks (warp_spec.h) for up to kSplitGrid workgroups.  Measured on
+    // MI355X against one workgroup per tile (RMSNorm + sinf, kernel time): 64 x 4
+    // KiB in 1 tile 65 -> 20 us, 128 x 16 KiB in 1 tile 279 -> 88, 1024 x 16
+    // KiB in 8 tiles 547 -> 367, 4096 x 16 KiB in 32 tiles 1301 -> 1224, 8192 x
+    // 16 KiB in 64 tiles 2453 -> 2425.  64 workgroups leave up to 5% more from
+    // 32 tiles on; 256 gain 1% on 512 KiB chunks but lose up to 5% on smaller ones.
+    static constexpr unsigned kSplitGrid = 128;
+    unsigned split_grid() const;
 
     // Wait for the launch to finish.  False if the kernel reported a stalled
     // hand-off or the stream returned an error.
@@ -317,7 +327,8 @@ template <typename KernelFn, typename ComputeFn>
 void gfd::WarpSpecSession::launch(KernelFn kernel, ComputeFn compute_fn, gfd_stream_t stream) {
     before_launch(stream);
     const LaunchParams p = get_launch_params();
-    hipLaunchKernelGGL(kernel, dim3(p.grid), dim3(p.block), 0, (hipStream_t)stream, p.tq, p.gpu_buffer, p.cpu_base,
+    const unsigned grid = warp_spec::_splits_chunks<ComputeFn>::value ? split_grid() : p.grid;
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(p.block), 0, (hipStream_t)stream, p.tq, p.gpu_buffer, p.cpu_base,
                        compute_fn);
 }
 

@@ -211,6 +211,39 @@ def test_warp_spec_rms_sin(total, ts, tile, chunk, db, blocks):
     assert (got[moved * 4:] == 0xCD).all()
 
 
+# (tiles, chunks per tile, double buffer, workgroups): parts of 1, 2, 3 and all
+# chunks; chunk counts that 2 does not divide; explicit grids of whole and
+# ragged multiples of the tiles; the most tiles that are still cut.
+@pytest.mark.parametrize("tiles,chunks,db,blocks", [(1, 1, False, 0), (1, 8, False, 0), (3, 4, True, 0), (2, 3, True, 0),
+                                                    (2, 6, False, 0), (5, 12, False, 0), (7, 4, True, 28),
+                                                    (7, 4, True, 30), (7, 4, False, 13), (33, 4, True, 0),
+                                                    (64, 4, True, 0), (65, 4, True, 0), (300, 2, True, 700)])
+def test_warp_spec_parts_of_tiles(tiles, chunks, db, blocks):
+    """Few tiles cut into parts for more workgroups (kSplitsChunks): every token
+    landed and reduced once, whole tiles counted, on two launches in a row."""
+    log("warp spec parts tiles=%d chunks=%d db=%d blocks=%d" % (tiles, chunks, db, blocks))
+    c, ts = 5, 1040
+    total, nf = tiles * chunks * c, ts // 4
+    host = gfd_amd.HostBuffer(total * ts)
+    host.array.view(np.float32)[:] = np.random.default_rng(total).standard_normal(total * nf, dtype=np.float32)
+    dst = gfd_amd.DeviceBuffer(total * ts + 64)
+    dst.fill(0xCD)
+    out = gfd_amd.DeviceBuffer(total * 4 + 64)
+    out.fill(0xCD)
+    res, _ = gfd_amd.warp_spec_run_rms_sin(host.ptr, dst.ptr, total, ts, out.ptr, chunks * c, c, db,
+                                           num_blocks=blocks, iters=2)
+    assert res["error_bits"] == 0 and res["lists_done"] == tiles and res["units_done"] == total
+    if blocks:
+        assert res["grid"] == blocks
+    landed = dst.download()
+    assert (landed[:total * ts] == host.array).all() and (landed[total * ts:] == 0xCD).all()
+    got = out.download()
+    want, mag = rms_sin_reference(host.array.view(np.float32).reshape(total, nf))
+    y = got[:total * 4].view(np.float32).astype(np.float64)
+    assert np.all(np.abs(y - want) <= 1e-4 * mag + 1e-6)
+    assert (got[total * 4:] == 0xCD).all()
+
+
 def test_warp_spec_rejects_oversized_block():
     host = gfd_amd.HostBuffer(4096 * 64)
     dst = gfd_amd.DeviceBuffer(4096 * 64)
