@@ -19,7 +19,7 @@
 // each list exactly once, on wave 1, as with the reference.
 //
 // A functor may instead take the rows of each list one by one, as the
-// transfer wave copies them, straight from an LDS ring of SG_ROW_SLOTS rows,
+// transfer wave copies them, straight from an LDS ring of SG_ROW_SLOTS slots,
 // by declaring `static constexpr bool kStagesRows = true` and
 //
 //   __device__ uint32_t staged_row_bytes() const;  // R: 1 .. 14 KiB in whole KiB (else: list mode)
@@ -27,8 +27,9 @@
 //
 // besides operator() (used when R is not a size the ring takes).  Entries of
 // exactly R bytes, 16-byte aligned on both sides, are then loaded by the
-// transfer wave, stored to HBM and written into the ring; compute wave c of C
-// gets the workgroup's staged rows c, c + C, ... in order.  Other entries are
+// transfer wave, stored to HBM and written into the ring, in groups of as many
+// rows as a slot takes (rows of more than 5 KiB one by one); compute wave c of
+// C gets the workgroup's groups c, c + C, ... in order, row by row.  Other entries are
 // copied as usual and not shown to the functor, and lists are still marked
 // done once all their bytes have landed.  The rows reach the compute waves
 // through LDS instead of being loaded again from HBM, so the compute waves
@@ -133,22 +134,32 @@ struct SGRowView {
     bool first;  // this wave's first row of the launch
     int* slot;
     // Hand the slot back to the transfer wave once data has been read (the
-    // workgroup-scope release waits for this wave's LDS reads).
+    // workgroup-scope release waits for this wave's LDS reads).  A slot of
+    // several rows is handed back with its last one (null before that).
     __device__ __forceinline__ void release() const {
-        if (lane_id == 0) __hip_atomic_store(slot, 0, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+        if (slot && lane_id == 0) __hip_atomic_store(slot, 0, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
 };
 
+// A ring slot holds a group of as many rows of V KiB as its 14 KiB take, loaded
+// together.  With one row at a time a transfer wave has V KiB in flight: 3380
+// rows of 1 KiB, normalised, took 184 us launch to end (floor 61), now 103; 2000
+// of 2 / 3 / 4 KiB 158 / 189 / 198, now 113 / 153 / 177.  From 6 KiB on two
+// rows are no faster than one (2000 of 7 KiB: 283 against 278).
+constexpr int SG_GROUP_ROWS = SG_MAX_STAGED_ROW / 1024;
+constexpr int _group_rows(int v) { return v <= 5 ? SG_GROUP_ROWS / v : 1; }
 struct _SGRowRing {
     wave::vec4u data[SG_ROW_SLOTS][SG_MAX_STAGED_ROW / 16];
-    uint64_t dst[SG_ROW_SLOTS];
-    uint32_t tag[SG_ROW_SLOTS], list_id[SG_ROW_SLOTS];
-    int flag[SG_ROW_SLOTS];  // r + 1 while the slot holds the workgroup's staged row r; 0 once free
+    uint64_t dst[SG_ROW_SLOTS][SG_GROUP_ROWS];
+    uint32_t tag[SG_ROW_SLOTS][SG_GROUP_ROWS], list_id[SG_ROW_SLOTS];
+    uint32_t rows[SG_ROW_SLOTS];
+    int flag[SG_ROW_SLOTS];  // g + 1 while the slot holds the workgroup's staged group g; 0 once free
 };
 struct _SGNoRowRing {
     wave::vec4u data[1][1];
-    uint64_t dst[1];
-    uint32_t tag[1], list_id[1];
+    uint64_t dst[1][1];
+    uint32_t tag[1][1], list_id[1];
+    uint32_t rows[1];
     int flag[1];
 };
 
@@ -342,15 +353,17 @@ __device__ __forceinline__ int _sg_copy_batches(_SGJob* job, const SGTaskQueue* 
     return nbatches;
 }
 
-// Transfer wave, staged rows of V KiB: copy the list's entries, staging each
-// row of exactly V KiB (16-byte aligned) into the next ring slot once its
-// compute wave has freed it; other entries are copied as they are.  Adds the
-// bytes copied; false if a slot was never freed (the compute waves stalled).
+// Transfer wave, staged rows of V KiB: copy the list's entries, staging the
+// rows of exactly V KiB (16-byte aligned) in groups into the next ring slot
+// once its compute wave has freed it; other entries are copied as they are.
+// Adds the bytes copied; false if a slot was never freed (the compute waves
+// stalled).
 template <int V>
 __device__ __forceinline__ bool _sg_stage_rows(const SGTaskQueue* ring, uint32_t pool_offset, uint32_t count,
-                                               uint32_t list_id, _SGRowRing* rr, int* nrows, uint64_t* bytes) {
+                                               uint32_t list_id, _SGRowRing* rr, int* ngroups, uint64_t* bytes) {
     using wave::vec4u;
     constexpr uint32_t kRow = (uint32_t)V * 1024;
+    constexpr int R = _group_rows(V);
     const int lane = wave::lane_id();
     for (uint32_t first = 0; first < count; first += wave::kWidth) {
         uint64_t md = 0, ms = 0, mn = 0;
@@ -372,28 +385,55 @@ __device__ __forceinline__ bool _sg_stage_rows(const SGTaskQueue* ring, uint32_t
             wave::copy<4>(wave::readlane64(md, j), wave::readlane64(ms, j), n);
             *bytes += n;
         }
-        for (uint64_t rows = __ballot(st); rows; rows &= rows - 1) {
-            const int j = __builtin_ctzll(rows);
-            const uint64_t s0 = wave::readlane64(ms, j), d0 = wave::readlane64(md, j);
-            const uint32_t tj = (uint32_t)__builtin_amdgcn_readlane((int)tag, j);
-            const int r = *nrows;
-            const int slot = r % SG_ROW_SLOTS;
-            if (!wave::wait_lds_eq(&rr->flag[slot], 0)) return false;
-            vec4u v[V];
+        for (uint64_t rows = __ballot(st); rows;) {
+            const int g = *ngroups;
+            const int slot = g % SG_ROW_SLOTS;
+            const int have = __builtin_popcountll(rows);
+            const int n = R == 1 ? 1 : (have < R ? have : R);
+            uint64_t s0[R], d0[R];
+            uint32_t tj[R];
 #pragma unroll
-            for (int k = 0; k < V; k++) v[k] = wave::gload(s0 + (uint64_t)(k * wave::kWidth + lane) * 16);
-#pragma unroll
-            for (int k = 0; k < V; k++) wave::gstore(d0 + (uint64_t)(k * wave::kWidth + lane) * 16, v[k]);
-#pragma unroll
-            for (int k = 0; k < V; k++) rr->data[slot][k * wave::kWidth + lane] = v[k];
-            if (lane == 0) {
-                rr->dst[slot] = d0;
-                rr->tag[slot] = tj;
-                rr->list_id[slot] = list_id;
-                wave::lds_store(&rr->flag[slot], r + 1);  // release: the row and its fields first
+            for (int i = 0; i < R; i++) {
+                // Past the group's rows: its first row's place in HBM is read
+                // instead (no host read, and the value is not kept), so that
+                // all loads stay straight-line code.
+                if (i < n) {
+                    const int j = __builtin_ctzll(rows);
+                    rows &= rows - 1;
+                    s0[i] = wave::readlane64(ms, j);
+                    d0[i] = wave::readlane64(md, j);
+                    tj[i] = (uint32_t)__builtin_amdgcn_readlane((int)tag, j);
+                } else {
+                    s0[i] = d0[i] = d0[0];
+                    tj[i] = 0;
+                }
             }
-            *nrows = r + 1;
-            *bytes += kRow;
+            if (!wave::wait_lds_eq(&rr->flag[slot], 0)) return false;
+            vec4u v[R * V];
+#pragma unroll
+            for (int k = 0; k < R * V; k++)
+                v[k] = wave::gload(s0[k / V] + (uint64_t)(k % V * wave::kWidth + lane) * 16);
+#pragma unroll
+            for (int i = 0; i < R; i++)
+                if (i < n) {
+#pragma unroll
+                    for (int k = 0; k < V; k++)
+                        wave::gstore(d0[i] + (uint64_t)(k * wave::kWidth + lane) * 16, v[i * V + k]);
+                }
+#pragma unroll
+            for (int k = 0; k < R * V; k++) rr->data[slot][k * wave::kWidth + lane] = v[k];
+            if (lane == 0) {
+#pragma unroll
+                for (int i = 0; i < R; i++) {
+                    rr->dst[slot][i] = d0[i];
+                    rr->tag[slot][i] = tj[i];
+                }
+                rr->list_id[slot] = list_id;
+                rr->rows[slot] = (uint32_t)n;
+                wave::lds_store(&rr->flag[slot], g + 1);  // release: the rows and their fields first
+            }
+            *ngroups = g + 1;
+            *bytes += (uint64_t)n * kRow;
         }
     }
     return true;
@@ -402,14 +442,14 @@ __device__ __forceinline__ bool _sg_stage_rows(const SGTaskQueue* ring, uint32_t
 // (Instantiated only for functors that stage rows.)
 template <bool kOn>
 __device__ __forceinline__ bool _sg_stage_rows_kb(uint32_t kb, const SGTaskQueue* ring, uint32_t pool_offset,
-                                                  uint32_t count, uint32_t list_id, _SGRowRing* rr, int* nrows,
+                                                  uint32_t count, uint32_t list_id, _SGRowRing* rr, int* ngroups,
                                                   uint64_t* bytes) {
     if constexpr (!kOn) {
         return false;
     } else {
         switch (kb) {
 #define GFD_SG_STAGE_CASE(n) \
-    case n: return _sg_stage_rows<n>(ring, pool_offset, count, list_id, rr, nrows, bytes);
+    case n: return _sg_stage_rows<n>(ring, pool_offset, count, list_id, rr, ngroups, bytes);
             GFD_SG_STAGE_CASE(1) GFD_SG_STAGE_CASE(2) GFD_SG_STAGE_CASE(3) GFD_SG_STAGE_CASE(4) GFD_SG_STAGE_CASE(5)
             GFD_SG_STAGE_CASE(6) GFD_SG_STAGE_CASE(7) GFD_SG_STAGE_CASE(8) GFD_SG_STAGE_CASE(9) GFD_SG_STAGE_CASE(10)
             GFD_SG_STAGE_CASE(11) GFD_SG_STAGE_CASE(12) GFD_SG_STAGE_CASE(13) GFD_SG_STAGE_CASE(14)
@@ -483,7 +523,7 @@ __device__ __forceinline__ void _sg_transfer_warp_loop(DescriptorQueue* dq, SGTa
         const uint64_t gpu_first =
             list_base + __hip_atomic_load(&cnt->host_lists, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         uint64_t nlists = 0;
-        int nrows = 0;  // rows staged (staged-row mode)
+        int ngroups = 0;  // groups of rows staged (staged-row mode)
         for (uint64_t iter = 0;; iter++) {
             const int s = (int)(iter & 1);
             if (has_compute && !staged && !wave::wait_lds_eq(&slots[s].free, 1)) {
@@ -509,7 +549,7 @@ __device__ __forceinline__ void _sg_transfer_warp_loop(DescriptorQueue* dq, SGTa
             uint64_t bytes = 0;
             if (staged) {
                 if (!_sg_stage_rows_kb<kStaging>(staged_bytes / 1024, ring, pool_offset, count, list_id,
-                                                 reinterpret_cast<_SGRowRing*>(&rr), &nrows, &bytes)) {
+                                                 reinterpret_cast<_SGRowRing*>(&rr), &ngroups, &bytes)) {
                     if (lane == 0)
                         __hip_atomic_fetch_or(&cnt->error, SG_ERR_SLOT_WAIT, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                     break;
@@ -621,7 +661,7 @@ __device__ __forceinline__ void _sg_transfer_warp_loop(DescriptorQueue* dq, SGTa
         }
     } else if (has_compute && staged && w >= 1 && w <= ncompute) {
         // ---------------- compute wave(s), staged rows: wave w takes the
-        // workgroup's staged rows w - 1, w - 1 + ncompute, ...; bounded like
+        // workgroup's staged groups w - 1, w - 1 + ncompute, ...; bounded like
         // the list-mode compute wave below.
         if constexpr (kStaging) {
             const uint64_t limit = _idle_limit_ticks(sq, cnt) + 100000000ull;
@@ -636,7 +676,7 @@ __device__ __forceinline__ void _sg_transfer_warp_loop(DescriptorQueue* dq, SGTa
                         ready = true;
                         break;
                     }
-                    if (wave::lds_load(&terminated)) {  // every row is staged by now: row i is here or never comes
+                    if (wave::lds_load(&terminated)) {  // every group is staged by now: group i is here or never comes
                         ready = wave::lds_load(&rr.flag[s]) == i + 1;
                         break;
                     }
@@ -650,16 +690,19 @@ __device__ __forceinline__ void _sg_transfer_warp_loop(DescriptorQueue* dq, SGTa
                 }
                 if (!ready) break;
                 SGRowView view;
-                view.data = rr.data[s];
-                view.dst = rr.dst[s];
                 view.bytes = staged_bytes;
-                view.tag = rr.tag[s];
                 view.list_id = rr.list_id[s];
                 view.lane_id = lane;
-                view.first = first;
-                view.slot = &rr.flag[s];
-                compute_fn.row(view);
-                first = false;
+                const int rows = __builtin_amdgcn_readfirstlane((int)rr.rows[s]);
+                for (int j = 0; j < rows; j++) {
+                    view.data = rr.data[s] + (uint32_t)j * (staged_bytes / 16);
+                    view.dst = rr.dst[s][j];
+                    view.tag = rr.tag[s][j];
+                    view.first = first;
+                    view.slot = j == rows - 1 ? &rr.flag[s] : nullptr;
+                    compute_fn.row(view);
+                    first = false;
+                }
             }
         }
     } else if (has_compute && w >= 1 && w <= ncompute) {

@@ -44,7 +44,10 @@ def run_session(m, sess, with_norm, rows_per_list, eps=1e-6):
                                                    (4096, 64, 7168, 2, 0, 1), (64, 8, 512, 4, 2, 1),
                                                    (300, 5, 1024, 7, 0, 1), (1000, 16, 2048, 1, 8, 1),
                                                    (4096, 64, 7168, 32, 0, 3), (4096, 64, 7168, 7, 4, 2),
-                                                   (300, 5, 1024, 1, 2, 3), (4096, 64, 7168, 48, 40, 3)])
+                                                   (300, 5, 1024, 1, 2, 3), (4096, 64, 7168, 48, 40, 3),
+                                                   # groups of 14, 4, 2 rows and single ones; short groups at list ends
+                                                   (700, 9, 512, 64, 3, 3), (333, 7, 1536, 13, 2, 2),
+                                                   (200, 5, 2560, 9, 4, 3), (150, 4, 3072, 5, 0, 1)])
 def test_moe_through_session(T, E, dim, rpl, blocks, cw):
     print("moe session T=%d E=%d dim=%d rows/list=%d blocks=%d compute waves=%d" % (T, E, dim, rpl, blocks, cw),
           flush=True)
