@@ -398,5 +398,6 @@ extern "C" int gfd_sg_session_launch_moe(gfd_sg_session_t s, const void* host_ba
         hipLaunchKernelGGL(sg_moe_kernel<NoCompute>, grid, block, 0, (hipStream_t)stream, p->get_desc_queue(),
                            p->get_sg_queue(), NoCompute{}, m, 2);
     const hipError_t e = hipGetLastError();
+    if (e == hipSuccess) p->after_launch();
     return e == hipSuccess ? 0 : fail(e, "gfd_sg_session_launch_moe: launch failed");
 }

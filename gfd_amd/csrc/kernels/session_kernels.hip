@@ -335,6 +335,21 @@ __global__ __launch_bounds__(256) void sg_prepare_kernel(uint64_t* d_list_done, 
     for (uint64_t k = i; k < trace_words; k += n) trace[k] = 0;
 }
 
+__global__ __launch_bounds__(256) void ws_prepare_kernel(uint64_t* d, uint64_t words) {
+    for (uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; k < words; k += (uint64_t)gridDim.x * blockDim.x)
+        d[k] = 0;
+}
+
+// A launch's progress and counters, to pinned memory behind it on its stream:
+// the host then finds them there once it has synchronised the stream, without
+// a copy of its own (hipMemcpy of some words takes 10-13 us).
+__global__ __launch_bounds__(256) void session_report_kernel(const uint64_t* src0, uint64_t* dst0, uint64_t n0,
+                                                            const uint64_t* src1, uint64_t* dst1, uint64_t n1) {
+    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x, n = (uint64_t)gridDim.x * blockDim.x;
+    for (uint64_t k = i; k < n0; k += n) dst0[k] = src0[k];
+    for (uint64_t k = i; k < n1; k += n) dst1[k] = src1[k];
+}
+
 int fail(int code, const char* what) {
     gfd_internal_set_error(what);
     return code ? code : (int)hipErrorInvalidValue;
@@ -426,6 +441,7 @@ int warp_spec_run(const void* cpu_src, void* gpu_dst, uint32_t total_tokens, uin
         }
         (void)hipEventRecord(e1, nullptr);
         const hipError_t le = hipGetLastError();
+        if (le == hipSuccess) s.after_launch();
         const bool ok = s.synchronize();
         float ms = 0.f;
         (void)hipEventElapsedTime(&ms, e0, e1);
@@ -527,6 +543,7 @@ extern "C" int gfd_sg_session_launch_gpu_submit(gfd_sg_session_t s, const gfd_de
         hipLaunchKernelGGL(sg_gpu_submit_kernel<NullList>, grid, block, 0, (hipStream_t)stream, p->get_desc_queue(),
                            p->get_sg_queue(), NullList{}, ents, entries_per_list, num_lists);
     const hipError_t e = hipGetLastError();
+    if (e == hipSuccess) p->after_launch();
     return e == hipSuccess ? 0 : fail(e, "gfd_sg_session_launch_gpu_submit: launch failed");
 }
 
@@ -537,6 +554,18 @@ extern "C" int gfd_sg_prepare_launch(uint64_t* d_list_done, const void* counters
     std::memcpy(&c, counters, sizeof(c));
     hipLaunchKernelGGL(sg_prepare_kernel, dim3(4), dim3(256), 0, (hipStream_t)stream, d_list_done, c, trace,
                        trace_words);
+    return (int)hipGetLastError();
+}
+
+extern "C" int gfd_ws_prepare_launch(uint64_t* d, uint64_t words, gfd_stream_t stream) {
+    hipLaunchKernelGGL(ws_prepare_kernel, dim3(4), dim3(256), 0, (hipStream_t)stream, d, words);
+    return (int)hipGetLastError();
+}
+
+extern "C" int gfd_session_report(const uint64_t* src0, uint64_t* dst0, uint64_t n0, const uint64_t* src1,
+                                  uint64_t* dst1, uint64_t n1, gfd_stream_t stream) {
+    hipLaunchKernelGGL(session_report_kernel, dim3(1), dim3(256), 0, (hipStream_t)stream, src0, dst0, n0, src1, dst1,
+                       n1);
     return (int)hipGetLastError();
 }
 

@@ -11,7 +11,9 @@
 #include <chrono>
 #include <cstddef>
 #include <cstring>
+#include <mutex>
 #include <thread>
+#include <vector>
 
 #include "gfd/log.h"
 #include "gfd/warp_spec_session.h"
@@ -48,9 +50,36 @@ CpuPollingThread* make_session_poller(DescriptorQueue* queue, void* gpu_base, vo
     return p;
 }
 
+// Queues that destroyed WarpSpecSessions left: allocating and freeing one (1
+// MiB pinned, and its first touch) took 72 us a session, clearing a kept one
+// takes 6.
+struct SpareQueue {
+    int device;
+    TiledQueue* tq;
+    uint64_t* signals;
+};
+std::mutex g_spare_mu;
+std::vector<SpareQueue> g_spare;
+
+constexpr size_t kTileWords = (size_t)MAX_TILES + TILE_DEVICE_COUNTER_WORDS;
+// Where the counters' copy lies behind a pinned queue of `bytes`.
+constexpr size_t report_offset(size_t bytes) { return (bytes + 63) & ~(size_t)63; }
+
 }  // namespace
 
 // ============================================================ WarpSpecSession
+
+void WarpSpecSession::release_spare_queues() {
+    std::vector<SpareQueue> all;
+    {
+        std::lock_guard<std::mutex> lock(g_spare_mu);
+        all.swap(g_spare);
+    }
+    for (const SpareQueue& q : all) {
+        gfd_hip_free(q.signals);
+        gfd_hip_host_free(q.tq);
+    }
+}
 
 WarpSpecSession::WarpSpecSession(const WarpSpecConfig& config) : config_(config) {
     // Validation as src/warp_spec_session.cpp:11-23, plus the wave64 block limit.
@@ -85,12 +114,27 @@ WarpSpecSession::WarpSpecSession(const WarpSpecConfig& config) : config_(config)
         config_.transfer_helper_waves =
             auto_helper_waves(std::min(num_blocks_, (int)std::max<uint32_t>(1, config_.total_tiles())));
 
-    void* q = nullptr;
-    if (gfd_hip_host_alloc(&q, sizeof(TiledQueue), GFD_HOST_COHERENT) != 0) {
-        GFD_LOG_ERROR("WarpSpecSession: TiledQueue allocation failed\n");
-        return;
+    gfd_hip_get_device(&device_);
+    {
+        std::lock_guard<std::mutex> lock(g_spare_mu);
+        for (size_t i = 0; i < g_spare.size(); i++) {
+            if (g_spare[i].device != device_) continue;
+            tq_ = g_spare[i].tq;
+            d_signals_ = g_spare[i].signals;
+            g_spare.erase(g_spare.begin() + (long)i);
+            break;
+        }
     }
-    tq_ = static_cast<TiledQueue*>(q);
+    if (!tq_) {
+        void* q = nullptr;
+        if (gfd_hip_host_alloc(&q, report_offset(sizeof(TiledQueue)) + sizeof(TileDeviceCounters),
+                               GFD_HOST_COHERENT) != 0) {
+            GFD_LOG_ERROR("WarpSpecSession: TiledQueue allocation failed\n");
+            return;
+        }
+        tq_ = static_cast<TiledQueue*>(q);
+    }
+    report_ = reinterpret_cast<uint64_t*>((char*)tq_ + report_offset(sizeof(TiledQueue)));
     std::memset((void*)tq_, 0, sizeof(TiledQueue));
     tq_->scheduler.total_tiles = config_.total_tiles();
     tq_->scheduler.tokens_per_tile = config_.tokens_per_tile;
@@ -98,14 +142,16 @@ WarpSpecSession::WarpSpecSession(const WarpSpecConfig& config) : config_(config)
     tq_->scheduler.chunks_per_tile = config_.chunks_per_tile();
     tq_->scheduler.token_size = config_.token_size;
 
-    const size_t words = (size_t)MAX_TILES + TILE_DEVICE_COUNTER_WORDS;
-    void* d = nullptr;
-    if (gfd_hip_malloc(&d, words * sizeof(uint64_t)) != 0) {
-        GFD_LOG_ERROR("WarpSpecSession: device signal allocation failed\n");
-        return;
+    if (!d_signals_) {
+        void* d = nullptr;
+        if (gfd_hip_malloc(&d, kTileWords * sizeof(uint64_t)) != 0) {
+            GFD_LOG_ERROR("WarpSpecSession: device signal allocation failed\n");
+            return;
+        }
+        d_signals_ = static_cast<uint64_t*>(d);
     }
-    d_signals_ = static_cast<uint64_t*>(d);
-    gfd_hip_memset_d8((uint64_t)(uintptr_t)d_signals_, 0, words * sizeof(uint64_t));
+    gfd_hip_memset_d8((uint64_t)(uintptr_t)d_signals_, 0, kTileWords * sizeof(uint64_t));
+    cleared_ = true;
     tq_->d_tile_chunk_done = d_signals_;
     ok_ = true;
 }
@@ -114,6 +160,17 @@ WarpSpecSession::~WarpSpecSession() {
     if (running_) synchronize();
     delete poller_;
     poller_ = nullptr;
+    // A kernel that the caller launched on this queue may still run: the
+    // queue changes hands only once the device is idle (as freeing it would
+    // wait for).
+    if (ok_ && gfd_hip_device_synchronize() == 0) {
+        std::lock_guard<std::mutex> lock(g_spare_mu);
+        if (g_spare.size() < (size_t)kSpareQueues) {
+            g_spare.push_back(SpareQueue{device_, tq_, d_signals_});
+            tq_ = nullptr;
+            d_signals_ = nullptr;
+        }
+    }
     if (d_signals_) gfd_hip_free(d_signals_);
     if (tq_) gfd_hip_host_free(tq_);
 }
@@ -139,9 +196,13 @@ unsigned WarpSpecSession::split_grid() const {
 void WarpSpecSession::reset() {
     if (running_) synchronize();
     if (!tq_) return;
-    if (d_signals_)
-        gfd_hip_memset_d8((uint64_t)(uintptr_t)d_signals_, 0,
-                          ((size_t)MAX_TILES + TILE_DEVICE_COUNTER_WORDS) * sizeof(uint64_t));
+    if (d_signals_) gfd_hip_memset_d8((uint64_t)(uintptr_t)d_signals_, 0, kTileWords * sizeof(uint64_t));
+    cleared_ = true;
+    clear_progress();
+}
+
+// reset() but for the words in HBM.
+void WarpSpecSession::clear_progress() {
     std::memset((void*)tq_->tile_chunk_done, 0, sizeof(tq_->tile_chunk_done));
     tq_->scheduler.next_tile = 0;
     error_bits_ = 0;
@@ -162,10 +223,30 @@ CpuPollingThread* WarpSpecSession::get_poller() const {
 }
 
 void WarpSpecSession::before_launch(gfd_stream_t stream) {
-    reset();  // as the reference's launch (warp_spec_session.h:217)
+    // reset(), as the reference's launch (warp_spec_session.h:217), with the
+    // words in HBM cleared on the launch's own stream, ahead of the kernel.
+    if (running_) synchronize();
+    if (ok_) {
+        // A stream of its own need not wait for the null stream's clear.
+        if (cleared_ && stream) gfd_hip_stream_synchronize(nullptr);
+        cleared_ = false;
+        if (gfd_ws_prepare_launch(d_signals_, kTileWords, stream) != 0) {
+            gfd_hip_memset_d8((uint64_t)(uintptr_t)d_signals_, 0, kTileWords * sizeof(uint64_t));
+            gfd_hip_device_synchronize();
+        }
+        clear_progress();
+    }
+    reported_ = false;
     stream_ = stream;
     launch_time_ = std::chrono::steady_clock::now();
     running_ = ok_;
+}
+
+void WarpSpecSession::after_launch() {
+    if (!running_) return;
+    reported_ = gfd_session_report(d_signals_, const_cast<uint64_t*>(tq_->tile_chunk_done),
+                                   std::min<uint32_t>(config_.total_tiles(), (uint32_t)MAX_TILES),
+                                   d_signals_ + MAX_TILES, report_, TILE_DEVICE_COUNTER_WORDS, stream_) == 0;
 }
 
 bool WarpSpecSession::synchronize() {
@@ -173,13 +254,25 @@ bool WarpSpecSession::synchronize() {
     const int rc = gfd_hip_stream_synchronize(stream_);
     last_elapsed_ms_ = ms_between(launch_time_, std::chrono::steady_clock::now());
     running_ = false;
+    // The counters and the host-visible progress mirror (tile_chunk_done,
+    // tiled_queue.h:41): after_launch() had them written, or one copy of both.
     TileDeviceCounters c{};
-    if (rc == 0 && gfd_hip_memcpy_d2h(&c, (uint64_t)(uintptr_t)(d_signals_ + MAX_TILES), sizeof(c)) == 0) {
+    const uint32_t n = std::min<uint32_t>(config_.total_tiles(), (uint32_t)MAX_TILES);
+    bool got = rc == 0 && reported_;
+    if (got) {
+        std::memcpy(&c, report_, sizeof(c));
+    } else if (rc == 0) {
+        std::vector<uint64_t> w(kTileWords);
+        got = gfd_hip_memcpy_d2h(w.data(), (uint64_t)(uintptr_t)d_signals_, kTileWords * sizeof(uint64_t)) == 0;
+        if (got) {
+            std::memcpy(&c, w.data() + MAX_TILES, sizeof(c));
+            std::memcpy((void*)tq_->tile_chunk_done, w.data(), n * sizeof(uint64_t));
+        }
+    }
+    reported_ = false;
+    if (got) {
         error_bits_ = c.error;
         tiles_done_ = c.tiles_done;
-        // Host-visible progress mirror (tile_chunk_done, tiled_queue.h:41).
-        const uint32_t n = std::min<uint32_t>(config_.total_tiles(), (uint32_t)MAX_TILES);
-        if (n) gfd_hip_memcpy_d2h((void*)tq_->tile_chunk_done, (uint64_t)(uintptr_t)d_signals_, n * sizeof(uint64_t));
         tq_->scheduler.next_tile = (uint32_t)std::min<uint64_t>(c.next_tile, config_.total_tiles());
         landed_tiles_total_ += tiles_done_;
         if (poller_) {
@@ -221,11 +314,12 @@ SGWarpSpecSession::SGWarpSpecSession(const SGWarpSpecConfig& config) : config_(c
     num_blocks_ = config_.num_blocks > 0 ? config_.num_blocks : std::min(default_num_blocks(), 64);
     if (config_.transfer_helper_waves < 0) config_.transfer_helper_waves = auto_helper_waves(num_blocks_);
     void* q = nullptr;
-    if (gfd_hip_host_alloc(&q, sizeof(SGTaskQueue), GFD_HOST_COHERENT) != 0) {
+    if (gfd_hip_host_alloc(&q, report_offset(sizeof(SGTaskQueue)) + sizeof(SGDeviceCounters), GFD_HOST_COHERENT) != 0) {
         GFD_LOG_ERROR("SGWarpSpecSession: SGTaskQueue allocation failed\n");
         return;
     }
     sq_ = static_cast<SGTaskQueue*>(q);
+    report_ = reinterpret_cast<uint64_t*>((char*)sq_ + report_offset(sizeof(SGTaskQueue)));
     std::memset((void*)sq_, 0, sizeof(SGTaskQueue));
     sq_->idle_limit_ms = config_.idle_limit_ms;
     if (gfd_hip_host_alloc(&q, sizeof(DescriptorQueue), GFD_HOST_COHERENT) != 0) {
@@ -384,9 +478,16 @@ void SGWarpSpecSession::before_launch(gfd_stream_t stream, int helper_waves, int
             error_bits_ |= 1ull << 63;
         }
     }
+    reported_ = false;
     stream_ = stream;
     launch_time_ = std::chrono::steady_clock::now();
     running_ = true;
+}
+
+void SGWarpSpecSession::after_launch() {
+    if (!running_) return;
+    reported_ = gfd_session_report(nullptr, nullptr, 0, reinterpret_cast<const uint64_t*>(sg_device_counters(sq_)),
+                                   report_, SG_DEVICE_COUNTER_WORDS, stream_) == 0;
 }
 
 bool SGWarpSpecSession::synchronize(uint64_t extra_gpu_lists) {
@@ -408,7 +509,11 @@ bool SGWarpSpecSession::synchronize(uint64_t extra_gpu_lists) {
     last_elapsed_ms_ = ms_between(launch_time_, std::chrono::steady_clock::now());
     running_ = false;
     SGDeviceCounters c{};
-    if (rc != 0 || gfd_hip_memcpy_d2h(&c, (uint64_t)(uintptr_t)sg_device_counters(sq_), sizeof(c)) != 0) {
+    const bool reported = rc == 0 && reported_;
+    reported_ = false;
+    if (reported) std::memcpy(&c, report_, sizeof(c));
+    if (rc != 0 ||
+        (!reported && gfd_hip_memcpy_d2h(&c, (uint64_t)(uintptr_t)sg_device_counters(sq_), sizeof(c)) != 0)) {
         GFD_LOG_ERROR("SGWarpSpecSession: synchronize failed: %s\n", gfd_hip_error_string(rc));
         error_bits_ |= 1ull << 63;
         return false;

@@ -67,6 +67,13 @@ extern "C" {
 // *counters, trace[0 .. trace_words) = 0.  A HIP error code, 0 on success.
 int gfd_sg_prepare_launch(uint64_t* d_list_done, const void* counters, uint64_t* trace, uint64_t trace_words,
                           gfd_stream_t stream);
+// The same for a WarpSpec launch: d[0 .. words) = 0.
+int gfd_ws_prepare_launch(uint64_t* d, uint64_t words, gfd_stream_t stream);
+// Stream-ordered read-back behind a session kernel: n0 words of src0 (HBM) to
+// dst0 (pinned host memory) and n1 of src1 to dst1, visible to the host once
+// the stream is synchronised.
+int gfd_session_report(const uint64_t* src0, uint64_t* dst0, uint64_t n0, const uint64_t* src1, uint64_t* dst1,
+                       uint64_t n1, gfd_stream_t stream);
 }
 
 extern "C" {

@@ -151,14 +151,28 @@ public:
     uint64_t error_bits() const { return error_bits_; }
     uint64_t tiles_done() const { return tiles_done_; }
 
-    // Internal: called by launch().
+    // Internal: called by launch() ahead of the kernel and behind it (without
+    // the second, synchronize() copies the results back itself).
     void before_launch(gfd_stream_t stream);
+    void after_launch();
+
+    // Sessions hand their queue (1 MiB of pinned host memory and its HBM
+    // words) on to the next one on the device: a destroyed session leaves it,
+    // with the device idle, to at most kSpareQueues spare ones, and a new one
+    // takes and clears one before it allocates.  Frees the spare ones.
+    static constexpr int kSpareQueues = 4;
+    static void release_spare_queues();
 
 private:
     WarpSpecConfig config_;
     TiledQueue* tq_ = nullptr;
     uint64_t* d_signals_ = nullptr;  // MAX_TILES progress words + TileDeviceCounters
+    uint64_t* report_ = nullptr;     // pinned, behind tq_: the counters after a launch (after_launch)
+    bool reported_ = false;
+    bool cleared_ = false;           // the words in HBM were last cleared on the null stream
+    int device_ = 0;                 // whose queue it is
     int num_blocks_ = 0;
+    void clear_progress();
     bool ok_ = false;
     bool running_ = false;  // launched, not yet synchronized
     gfd_stream_t stream_ = nullptr;
@@ -252,6 +266,9 @@ public:
     // come from GPU submitters; see SGDeviceCounters::deadline).
     void before_launch(gfd_stream_t stream, int helper_waves = -1, int compute_waves = -1,
                        uint32_t deadline_ms = 0, SGTaskQueue* gpu_ring = nullptr);
+    // Internal: called behind the kernel (without it, synchronize() copies the
+    // counters back itself).
+    void after_launch();
     // An SGTaskQueue in HBM for GPU-submitted lists (allocated on first call;
     // nullptr if that fails).  A launch whose GPU submitters post there
     // passes it to before_launch as gpu_ring (SGDeviceCounters::dev_ring).
@@ -295,6 +312,8 @@ private:
 
     SGWarpSpecConfig config_;
     SGTaskQueue* sq_ = nullptr;
+    uint64_t* report_ = nullptr;  // pinned, behind sq_: the counters after a launch (after_launch)
+    bool reported_ = false;
     SGTaskQueue* dev_ring_ = nullptr;  // HBM: lists posted by GPU submitters
     DescriptorQueue* dq_ = nullptr;
     int num_blocks_ = 0;
@@ -330,6 +349,7 @@ void gfd::WarpSpecSession::launch(KernelFn kernel, ComputeFn compute_fn, gfd_str
     const unsigned grid = warp_spec::_splits_chunks<ComputeFn>::value ? split_grid() : p.grid;
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(p.block), 0, (hipStream_t)stream, p.tq, p.gpu_buffer, p.cpu_base,
                        compute_fn);
+    if (hipPeekAtLastError() == hipSuccess) after_launch();
 }
 
 template <typename KernelFn, typename ComputeFn>
@@ -337,5 +357,6 @@ void gfd::SGWarpSpecSession::launch(KernelFn kernel, ComputeFn compute_fn, gfd_s
     before_launch(stream);
     hipLaunchKernelGGL(kernel, dim3(num_blocks_), dim3(config_.block_size()), 0, (hipStream_t)stream, dq_, sq_,
                        compute_fn);
+    if (hipPeekAtLastError() == hipSuccess) after_launch();
 }
 #endif

@@ -8,6 +8,8 @@ GPU wave)."""
 import ctypes
 import sys
 
+from concurrent.futures import ThreadPoolExecutor
+
 import numpy as np
 import pytest
 
@@ -242,6 +244,32 @@ def test_warp_spec_parts_of_tiles(tiles, chunks, db, blocks):
     y = got[:total * 4].view(np.float32).astype(np.float64)
     assert np.all(np.abs(y - want) <= 1e-4 * mag + 1e-6)
     assert (got[total * 4:] == 0xCD).all()
+
+
+def test_warp_spec_queues_are_handed_on():
+    """A session takes a queue that an earlier one left and clears it: sessions
+    of other sizes in turn, and in four threads at once (more than one queue
+    in use, each its own), every launch whole and byte-exact."""
+    log("warp spec queues handed on")
+    shapes = [(1024, 4096, 128, 32), (64, 1024, 64, 16), (2000, 512, 100, 25), (128, 16384, 128, 32)]
+
+    def run(k, rounds):
+        total, ts, tile, chunk = shapes[k]
+        host = gfd_amd.HostBuffer(total * ts)
+        host.array.view(np.float32)[:] = np.random.default_rng(k).standard_normal(total * ts // 4, dtype=np.float32)
+        out = gfd_amd.DeviceBuffer(total * 4)
+        for _ in range(rounds):
+            dst = gfd_amd.DeviceBuffer(total * ts)
+            dst.fill(0)
+            res, _ = gfd_amd.warp_spec_run_rms_sin(host.ptr, dst.ptr, total, ts, out.ptr, tile, chunk, True)
+            assert res["error_bits"] == 0 and res["lists_done"] == total // tile
+            assert (dst.download() == host.array).all()
+        return True
+
+    for k in (0, 1, 2, 3, 1, 0):
+        assert run(k, 1)
+    with ThreadPoolExecutor(4) as ex:
+        assert all(ex.map(lambda k: run(k, 4), range(4)))
 
 
 def test_warp_spec_rejects_oversized_block():
