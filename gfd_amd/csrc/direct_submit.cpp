@@ -46,6 +46,13 @@ void direct_chunk(void* p, int chunk, size_t off, size_t len) {
 }
 
 constexpr size_t kContiguousSplitMin = 8u << 20;  // split one contiguous copy above this
+// Few destination runs: the zero-copy kernel above this many runs or above
+// direct_zc_min_bytes_, else a staged gather with an SDMA copy per run, which
+// starts sooner but takes 1.7 us per run.  Measured on MI355X, copies against
+// kernel: 4 runs of 4 KiB 11.3 / 13.2 us, 8 of 4 KiB 18.9 / 13.1, 41 of 10 KB
+// 87.4 / 20.4, 2 of 32 KiB 12.4 / 13.2, 6 of up to 50 KB 22.1 / 16.3, 2 of 1
+// MiB 53.4 / 48.9, 60 of up to 100 KB 148 / 74.
+constexpr int kKernelRuns = 5;
 constexpr int kZcNotTaken = INT_MIN;               // direct_zero_copy: the list does not qualify
 
 }  // namespace
@@ -344,15 +351,18 @@ int CpuPollingThread::zc_launch_head(const SGEntry* entries, int k, bool uniform
 // destination.  Sources that are pinned host memory are read in place;
 // otherwise the gather pool first packs them into the (pinned) direct staging
 // and the kernel reads from there.  The entry table goes to pinned memory the
-// kernel reads.  Returns 0 or an error code.
-int CpuPollingThread::direct_scattered(const SGEntry* entries, int count, size_t total, bool uniform) {
+// kernel reads.  Returns 0 or an error code.  required = false (few runs, which
+// SDMA copies can serve too): kZcNotTaken where a source is not pinned or a
+// destination is not device memory.
+int CpuPollingThread::direct_scattered(const SGEntry* entries, int count, size_t total, bool uniform, bool required) {
     if (zc_table_cap_ < count) {
         if (zc_table_) gfd_hip_host_free(zc_table_);
         zc_table_ = nullptr;
         zc_table_cap_ = 0;
         const int cap = std::max(count, 4096);
         void* t = nullptr;
-        if (gfd_hip_host_alloc(&t, (size_t)cap * sizeof(SGEntry), GFD_HOST_DEFAULT) != 0) return -1;
+        if (gfd_hip_host_alloc(&t, (size_t)cap * sizeof(SGEntry), GFD_HOST_DEFAULT) != 0)
+            return required ? -1 : kZcNotTaken;
         zc_table_ = static_cast<SGEntry*>(t);
         zc_table_cap_ = cap;
     }
@@ -367,6 +377,7 @@ int CpuPollingThread::direct_scattered(const SGEntry* entries, int count, size_t
         if (a < dlo || b > dhi) {
             uint64_t base = 0, size = 0;
             if (!gfd_hip_device_range(a, &base, &size) || b > base + size) {
+                if (!required) return kZcNotTaken;
                 GFD_LOG_ERROR("submit_direct: destination %d is not inside a device allocation\n", i);
                 return -1;
             }
@@ -376,8 +387,12 @@ int CpuPollingThread::direct_scattered(const SGEntry* entries, int count, size_t
         if (pinned && !direct_ce_manager_.host_source_ok(entries[i].src, entries[i].size)) pinned = false;
     }
     if (!any) return 0;  // nothing to move
+    if (!required && (!pinned || !zc_ready())) return kZcNotTaken;
+    bool cut = false;
+    int n = count;
     if (pinned) {
-        std::memcpy(zc_table_, entries, (size_t)count * sizeof(SGEntry));
+        static const int kWaves = gfd_zero_copy_target_waves();
+        n = zc_fill_sg_table(entries, count, total, zc_table_, zc_table_cap_, &cut, cut_waves(count, kWaves));
     } else {
         if (!direct_staging_ || total > direct_staging_size_ || !gather_) return -1;
         {
@@ -393,9 +408,12 @@ int CpuPollingThread::direct_scattered(const SGEntry* entries, int count, size_t
     }
     if (!zc_ready()) return -1;
     const uint64_t gen = ++zc_gen_;
-    int rc = gfd_zero_copy_gather_signal(reinterpret_cast<const gfd_sg_entry*>(zc_table_), count, zc_counter_,
-                                         zc_done_, gen, zc_stream_);
-    if (rc == 0) rc = zc_wait(gen);
+    int rc = (cut ? gfd_zero_copy_gather_signal_presliced : gfd_zero_copy_gather_signal)(
+        reinterpret_cast<const gfd_sg_entry*>(zc_table_), n, zc_counter_, zc_done_, gen, zc_stream_);
+    if (rc != 0) return rc;
+    trace(TRACE_ZC_LAUNCH, (uint32_t)count, total);
+    rc = zc_wait(gen);
+    trace(TRACE_ZC_DONE, 0, gen);
     return rc;
 }
 
@@ -547,14 +565,19 @@ double CpuPollingThread::submit_direct(const SGEntry* entries, int count) {
         // Destinations in several runs: a packed gather with one copy per run
         // piece, or the zero-copy kernel when there are many runs.
         const int nr = dst_runs(entries, count, kMaxRunCopies, direct_runs_);
-        if (nr <= kMaxRunCopies && direct_staging_ && total <= direct_staging_size_) {
+        if (nr <= kMaxRunCopies && (nr > kKernelRuns || total > direct_zc_min_bytes_) &&
+            total <= direct_zc_max_bytes_ && zc_pinned != 0 &&
+            (err = direct_scattered(entries, count, total, uniform, false)) != kZcNotTaken) {
+            // done by the zero-copy kernel (err 0) or failed
+        } else if (nr <= kMaxRunCopies && direct_staging_ && total <= direct_staging_size_) {
+            err = 0;
             std::lock_guard<std::mutex> lock(gather_mutex_);
             RunCopyCtx ctx{this, &direct_ce_manager_, direct_staging_, direct_runs_.data(), nr, 0, nch, 0, 0};
             gather_->run(entries, count, total, direct_staging_, direct_chunk_bytes_, run_copy_chunk, &ctx,
                          uniform ? 1 : 0);
             err = ctx.err;
         } else if (nr > kMaxRunCopies) {
-            err = direct_scattered(entries, count, total, uniform);
+            err = direct_scattered(entries, count, total, uniform, true);
         } else {
             err = direct_ce_manager_.submit_scatter_gather(entries, count);
         }

@@ -85,6 +85,22 @@ def blocks_layout(n, t, nblocks, gap):
     return offs, nblocks * (per * t + gap)
 
 
+# Either side of the lines between the SDMA copies and the kernel: 5 runs, 64
+# KiB, 64 runs, 8 MiB; pageable sources stay on the copies.
+@pytest.mark.parametrize("n,t,nblocks", [(4, 4096, 4), (5, 4096, 5), (6, 4096, 6), (2, 32768, 2), (2, 32784, 2),
+                                         (16, 1000, 16), (41, 10169, 41), (64, 100, 64), (65, 100, 65),
+                                         (8, 1 << 20, 8), (9, 1 << 20, 9), (700, 900, 7)])
+@pytest.mark.parametrize("pageable", [False, True])
+def test_direct_short_lists_of_runs(direct_poller, n, t, nblocks, pageable):
+    log("direct short runs n=%d t=%d blocks=%d pageable=%d" % (n, t, nblocks, pageable))
+    offs, region = blocks_layout(n, t, nblocks, 48)
+    c = Case(n, t, offs, region, pageable)
+    for _ in range(2):
+        c.dst.fill(SENTINEL)
+        assert direct_poller.submit_direct(c.entries, n) > 0
+        c.check()
+
+
 @pytest.mark.parametrize("n,t,nblocks", [(4096, 4096, 10), (2048, 1000, 64), (300, 4096, 2), (8192, 4096, 40)])
 def test_direct_few_runs(direct_poller, n, t, nblocks):
     log("direct few runs n=%d t=%d blocks=%d" % (n, t, nblocks))
