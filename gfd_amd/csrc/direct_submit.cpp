@@ -46,13 +46,15 @@ void direct_chunk(void* p, int chunk, size_t off, size_t len) {
 }
 
 constexpr size_t kContiguousSplitMin = 8u << 20;  // split one contiguous copy above this
-// Few destination runs: the zero-copy kernel above this many runs or above
-// direct_zc_min_bytes_, else a staged gather with an SDMA copy per run, which
-// starts sooner but takes 1.7 us per run.  Measured on MI355X, copies against
+// Short lists over few destination runs (at most kKernelRunEntries entries;
+// longer ones have long runs, which the copies carry well): the zero-copy
+// kernel above kKernelRuns runs or above direct_zc_min_bytes_, else a staged
+// gather with an SDMA copy per run, which starts sooner but takes 1.7 us per
+// run.  Measured on MI355X, copies against
 // kernel: 4 runs of 4 KiB 11.3 / 13.2 us, 8 of 4 KiB 18.9 / 13.1, 41 of 10 KB
 // 87.4 / 20.4, 2 of 32 KiB 12.4 / 13.2, 6 of up to 50 KB 22.1 / 16.3, 2 of 1
 // MiB 53.4 / 48.9, 60 of up to 100 KB 148 / 74.
-constexpr int kKernelRuns = 5;
+constexpr int kKernelRuns = 5, kKernelRunEntries = 2 * kMaxRunCopies;
 constexpr int kZcNotTaken = INT_MIN;               // direct_zero_copy: the list does not qualify
 
 }  // namespace
@@ -120,8 +122,8 @@ void run_copy_chunk(void* p, int chunk, size_t off, size_t len) {
     c->self->trace(CpuPollingThread::TRACE_CHUNK, (uint32_t)chunk, len);
 }
 
-// Zero-copy completion state: the HBM wave counter and the host word the
-// grid's last wave raises (allocated once per poller).
+// Zero-copy completion state: the HBM workgroup counter and the host word the
+// grid's last workgroup raises (allocated once per poller).
 bool CpuPollingThread::zc_ready() {
     if (zc_done_ && zc_counter_ && zc_stream_) return true;
     if (!zc_stream_ && gfd_hip_stream_create(&zc_stream_) != 0) return false;
@@ -242,7 +244,7 @@ bool CpuPollingThread::zc_dst_in_device(uint64_t lo, uint64_t hi) {
 }
 
 // Small destination-contiguous list with pinned sources: the zero-copy
-// kernel reads the tokens over PCIe and writes them to HBM; its last wave
+// kernel reads the tokens over PCIe and writes them to HBM; its last workgroup
 // raises zc_done_.  Uniform lists pass only their source addresses (8 bytes
 // per token); others pass the whole entry table.  Returns 0, kZcNotTaken
 // when the list does not qualify (the caller then takes the staged route), or
@@ -565,8 +567,8 @@ double CpuPollingThread::submit_direct(const SGEntry* entries, int count) {
         // Destinations in several runs: a packed gather with one copy per run
         // piece, or the zero-copy kernel when there are many runs.
         const int nr = dst_runs(entries, count, kMaxRunCopies, direct_runs_);
-        if (nr <= kMaxRunCopies && (nr > kKernelRuns || total > direct_zc_min_bytes_) &&
-            total <= direct_zc_max_bytes_ && zc_pinned != 0 &&
+        if (nr <= kMaxRunCopies && count <= kKernelRunEntries &&
+            (nr > kKernelRuns || total > direct_zc_min_bytes_) && total <= direct_zc_max_bytes_ && zc_pinned != 0 &&
             (err = direct_scattered(entries, count, total, uniform, false)) != kZcNotTaken) {
             // done by the zero-copy kernel (err 0) or failed
         } else if (nr <= kMaxRunCopies && direct_staging_ && total <= direct_staging_size_) {

@@ -280,7 +280,9 @@ int short_list_waves() { return std::max(4, env_int(kGatherShape.waves_env, kGat
 // the same on small ones, 384 and 512 no faster.  With a completion signal
 // every workgroup writes its L2 back, so there 64 waves (kGatherShape) stand:
 // submit_direct of 1024 x 4 KiB into scattered pages 89 us against 92.
-constexpr int kSgUnits = 1024;
+// At most 32 entries keep 64 waves: 32 of up to 70 KB 27.2 against 28.0 us, one
+// of 1 MiB alone 24.7 against 26.0.
+constexpr int kSgUnits = 1024, kShortSg = 32;
 constexpr ShapeDefaults kSgShape{kBytesPerWave, kMaxWaves, kMaxWaves, kDefaultUnroll, "GFD_ZC_WAVES", "GFD_ZC_UNROLL"};
 
 // slice: the table is the caller's list as it is.  Without it, each record is
@@ -291,7 +293,7 @@ int launch_gather_sg(const gfd_sg_entry* entries, int count, void* stream, GridD
     if (count == 0) return 0;
     const uint32_t pieces = slice && 2 * (int64_t)count <= kSgUnits ? (uint32_t)(kSgUnits / count) : 1u;
     const Shape s = shape_for((uint64_t)count * pieces, (uint64_t)count * pieces * 4096,
-                              done.host_word && slice ? kGatherShape : kSgShape);
+                              slice && (done.host_word || count <= kShortSg) ? kGatherShape : kSgShape);
     if (s.lds)
         hipLaunchKernelGGL(zc_gather_sg<true>, dim3(s.blocks), dim3(kBlock), 0, (hipStream_t)stream, entries,
                            (uint32_t)count, pieces, s.per_wave, s.unroll, done);

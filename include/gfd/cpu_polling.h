@@ -342,8 +342,8 @@ private:
     SGEntry* zc_table_ = nullptr;
     int zc_table_cap_ = 0;
     gfd_stream_t zc_stream_ = nullptr;
-    // Completion of the zero-copy kernels, signalled by the grid's last wave:
-    // a wave counter in HBM and the generation word it writes to host memory.
+    // Completion of the zero-copy kernels, signalled by the grid's last
+    // workgroup: a counter in HBM and the generation word it writes to host memory.
     unsigned int* zc_counter_ = nullptr;
     uint64_t* zc_done_ = nullptr;
     uint64_t zc_gen_ = 0;

@@ -200,7 +200,7 @@ int gfd_zero_copy_gather(const gfd_sg_entry* entries, int count, void* stream);
 /* The same three kernels with completion signalled to the host instead of by
  * the stream (no reference counterpart; the reference waits on stream events):
  * when every byte has landed (and is visible to any agent), the grid's last
- * wave stores done_value to *done_word (pinned host memory, ideally coherent),
+ * workgroup stores done_value to *done_word (pinned host memory, ideally coherent),
  * which the caller polls.  done_counter: one unsigned int in HBM, 0 before the
  * first launch; the kernel leaves it 0 again.  Launches that share a counter
  * must be ordered (one stream).  The stream still orders the launch as usual. */
