@@ -49,12 +49,16 @@ constexpr uint64_t kBytesPerWave = 128 * 1024;
 constexpr int kMinWaves = 64, kMaxWaves = 256;
 constexpr int kDefaultUnroll = 4;
 constexpr int kDefaultLds = 0;
-// Offload (HBM -> host): the stores are posted PCIe writes, so few waves fill
-// the link.  Measured on MI355X over 16-512 waves and U = 4/8/16: 8192 x 4 KiB
-// is flat at 54.8-54.9 GB/s from 16 to 128 waves and 54.5 at 256-512;
-// 2048 x 64 KiB peaks at 64 waves (55.5 GB/s).  One wave per 512 KiB, 16-64.
-constexpr uint64_t kScatterBytesPerWave = 512 * 1024;
-constexpr int kScatterMinWaves = 16, kScatterMaxWaves = 64;
+// Offload (HBM -> host): the stores are posted PCIe writes, but each wave's
+// loads are a round trip of their own.  128 waves up to 32 MiB, U = 8.
+// Measured on MI355X over 16-256 waves and U = 4/8/16, against one wave per
+// 512 KiB (16-64): 500 x 3333 B 46.4 -> 35.0 us, 2048 x 2 KiB 85.6 -> 79.7, 2 x
+// 1 MiB 48.3 -> 41.1, 2048 x 512 B 23.8 -> 22.2, 4096 x 3000 B 237 -> 233;
+// 8192 x 4 KiB the same (607).  Larger jobs keep 64 waves (2048 x 64 KiB 2414
+// us, 2419 with 128), and 256 lose 1% from 32 MiB on.  With a completion
+// signal every workgroup writes its L2 back: there the old 16-64 stand.
+constexpr uint64_t kScatterBytesPerWave = 512 * 1024, kScatterWideBytes = 32ull << 20;
+constexpr int kScatterMinWaves = 16, kScatterMaxWaves = 64, kScatterWideWaves = 128;
 constexpr int kScatterUnroll = 8;
 // Smallest piece a token is cut into when a list has too few tokens for its waves.
 constexpr int kMinPiece = 4096;
@@ -191,6 +195,8 @@ constexpr ShapeDefaults kGatherShape{kBytesPerWave, kMinWaves, kMaxWaves, kDefau
                                      "GFD_ZC_UNROLL"};
 constexpr ShapeDefaults kScatterShape{kScatterBytesPerWave, kScatterMinWaves, kScatterMaxWaves, kScatterUnroll,
                                       "GFD_ZCS_WAVES", "GFD_ZCS_UNROLL"};
+constexpr ShapeDefaults kScatterWideShape{kScatterBytesPerWave, kScatterWideWaves, kScatterWideWaves, kScatterUnroll,
+                                          "GFD_ZCS_WAVES", "GFD_ZCS_UNROLL"};
 
 // n entries of total_bytes.  token_size != 0: the entries are tokens of that
 // size, which may be cut into pieces: a list of fewer tokens than the target
@@ -254,7 +260,10 @@ int launch_scatter_tokens(const uint64_t* dst_addrs, const void* src, uint32_t t
         return (int)hipErrorInvalidValue;
     if (num_tokens == 0) return 0;
     if ((uint64_t)token_size >= (1ull << 30)) return (int)hipErrorInvalidValue;  // 1 GiB per token at most
-    const Shape s = shape_for((uint64_t)num_tokens, (uint64_t)num_tokens * token_size, kScatterShape, token_size);
+    const uint64_t total = (uint64_t)num_tokens * token_size;
+    const Shape s = shape_for((uint64_t)num_tokens, total,
+                              !done.host_word && total <= kScatterWideBytes ? kScatterWideShape : kScatterShape,
+                              token_size);
     if (s.lds)
         hipLaunchKernelGGL(zc_scatter_tokens<true>, dim3(s.blocks), dim3(kBlock), 0, (hipStream_t)stream, dst_addrs,
                            (uint64_t)(uintptr_t)src, token_size, (uint32_t)num_tokens, s.piece_shift, s.per_wave,
