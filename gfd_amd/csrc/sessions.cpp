@@ -61,6 +61,16 @@ struct SpareQueue {
 std::mutex g_spare_mu;
 std::vector<SpareQueue> g_spare;
 
+// Waits until `device` is idle; the current device stays what it was.
+bool device_idle(int device) {
+    int current = -1;
+    if (gfd_hip_get_device(&current) != 0) return false;
+    if (current == device) return gfd_hip_device_synchronize() == 0;
+    if (gfd_hip_set_device(device) != 0) return false;
+    const int rc = gfd_hip_device_synchronize();
+    return gfd_hip_set_device(current) == 0 && rc == 0;
+}
+
 constexpr size_t kTileWords = (size_t)MAX_TILES + TILE_DEVICE_COUNTER_WORDS;
 // Where the counters' copy lies behind a pinned queue of `bytes`.
 constexpr size_t report_offset(size_t bytes) { return (bytes + 63) & ~(size_t)63; }
@@ -161,9 +171,9 @@ WarpSpecSession::~WarpSpecSession() {
     delete poller_;
     poller_ = nullptr;
     // A kernel that the caller launched on this queue may still run: the
-    // queue changes hands only once the device is idle (as freeing it would
-    // wait for).
-    if (ok_ && gfd_hip_device_synchronize() == 0) {
+    // queue changes hands only once its device is idle (as freeing it would
+    // wait for), whichever device is current here.
+    if (ok_ && device_idle(device_)) {
         std::lock_guard<std::mutex> lock(g_spare_mu);
         if (g_spare.size() < (size_t)kSpareQueues) {
             g_spare.push_back(SpareQueue{device_, tq_, d_signals_});

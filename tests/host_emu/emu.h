@@ -2,8 +2,8 @@
 // Host-only emulation of the two runtime layers the poller stack calls (the
 // HSA runtime used by SdmaQueue and the gfd_hip_* shim), so that the product
 // sources cpu_polling.cpp, copy_engine.cpp, sdma.cpp, gather_engine.cpp,
-// staging_pool.cpp and direct_submit.cpp run unchanged on a machine without a
-// GPU.  Test infrastructure only: nothing here is linked into libgfd_amd.so.
+// staging_pool.cpp, direct_submit.cpp and sessions.cpp run unchanged on a
+// machine without a GPU.  Test infrastructure only: nothing here is linked into libgfd_amd.so.
 //
 // Copy engines are modelled the way the SDMA engines execute the packets the
 // HSA runtime writes for hsa_amd_memory_async_copy[_on_engine]:
@@ -42,6 +42,14 @@ unsigned zero_copy_launches();
 // Aborts the process, as a GPU page fault would end it, unless [p, p + n) is
 // pinned host memory or device memory (n = 0 passes).
 void require_gpu_access(const void* p, size_t n, const char* what);
+
+// GPUs the shim shows (1 unless a scenario asks for more); allocations belong
+// to the device that was current.  A kernel of a scenario's own "runs" on a
+// device from start_kernel until that device is synchronised: device_synchronize
+// of the current one, or a free of device memory there.
+void set_device_count(int n);
+void start_kernel(int device);
+bool kernel_runs(int device);
 
 // Engine stall watchdog: an engine that has polled one dependency for longer
 // than this (GFD_EMU_STALL_MS, default 5000) prints what it waits on and ends

@@ -19,7 +19,13 @@ struct Alloc {
     size_t size;
     Kind kind;
     uintptr_t agent_base;
+    int device;
 };
+
+constexpr int kMaxDevices = 4;
+int g_devices = 1;
+thread_local int t_device = 0;  // the thread's current device, as in HIP
+std::atomic<bool> g_kernel[kMaxDevices];
 
 std::mutex& reg_mu() {
     static std::mutex m;
@@ -35,12 +41,12 @@ std::map<uintptr_t, Alloc>& reg() {
 
 void note_alloc(void* p, size_t n, Kind k) {
     std::lock_guard<std::mutex> g(reg_mu());
-    reg()[(uintptr_t)p] = Alloc{n, k, (uintptr_t)p};
+    reg()[(uintptr_t)p] = Alloc{n, k, (uintptr_t)p, t_device};
 }
 
 void note_locked(void* p, size_t n, uintptr_t agent_base) {
     std::lock_guard<std::mutex> g(reg_mu());
-    reg()[(uintptr_t)p] = Alloc{n, Kind::Locked, agent_base};
+    reg()[(uintptr_t)p] = Alloc{n, Kind::Locked, agent_base, t_device};
 }
 
 uintptr_t locked_agent_base(uintptr_t base) {
@@ -51,8 +57,15 @@ uintptr_t locked_agent_base(uintptr_t base) {
 
 void note_free(void* p) {
     std::lock_guard<std::mutex> g(reg_mu());
-    reg().erase((uintptr_t)p);
+    const auto it = reg().find((uintptr_t)p);
+    if (it == reg().end()) return;
+    if (it->second.kind == Kind::Device) g_kernel[it->second.device] = false;
+    reg().erase(it);
 }
+
+void set_device_count(int n) { g_devices = n; }
+void start_kernel(int device) { g_kernel[device] = true; }
+bool kernel_runs(int device) { return g_kernel[device]; }
 
 bool find_alloc(const void* p, size_t n, Kind k, uintptr_t* base, size_t* size) {
     std::lock_guard<std::mutex> g(reg_mu());
@@ -108,15 +121,22 @@ unsigned zero_copy_launches() { return g_zc_launches.load(); }
 extern "C" {
 
 int gfd_hip_device_count(int* n) {
-    *n = 1;
+    *n = emu::g_devices;
     return 0;
 }
 int gfd_hip_get_device(int* dev) {
-    *dev = 0;
+    *dev = emu::t_device;
     return 0;
 }
-int gfd_hip_set_device(int dev) { return dev == 0 ? 0 : 101; }
-int gfd_hip_device_synchronize(void) { return 0; }
+int gfd_hip_set_device(int dev) {
+    if (dev < 0 || dev >= emu::g_devices) return 101;
+    emu::t_device = dev;
+    return 0;
+}
+int gfd_hip_device_synchronize(void) {
+    emu::g_kernel[emu::t_device] = false;
+    return 0;
+}
 int gfd_hip_pci_bus_id(char* buf, int len, int dev) {
     if (dev != 0) return 101;
     std::snprintf(buf, (size_t)len, "0000:c1:00.0");
@@ -215,6 +235,19 @@ int gfd_hip_device_range(uint64_t ptr, uint64_t* base, uint64_t* size) {
     *base = b;
     *size = s;
     return 1;
+}
+
+// The sessions' set-up and read-back kernels, on the calling thread.
+int gfd_ws_prepare_launch(uint64_t* d, uint64_t words, gfd_stream_t) {
+    std::memset(d, 0, words * sizeof(uint64_t));
+    return 0;
+}
+int gfd_sg_prepare_launch(uint64_t*, const void*, uint64_t*, uint64_t, gfd_stream_t) { return 801; }
+int gfd_session_report(const uint64_t* src0, uint64_t* dst0, uint64_t n0, const uint64_t* src1, uint64_t* dst1,
+                       uint64_t n1, gfd_stream_t) {
+    if (n0) std::memcpy(dst0, src0, n0 * sizeof(uint64_t));
+    if (n1) std::memcpy(dst1, src1, n1 * sizeof(uint64_t));
+    return 0;
 }
 
 // The Direct path's zero-copy route is a GPU kernel: not emulated.

@@ -1,5 +1,5 @@
 """The product poller stack on the CPU: gfd_amd/csrc/{cpu_polling,copy_engine,
-sdma,gather_engine,staging_pool,direct_submit}.cpp built unchanged with g++
+sdma,gather_engine,staging_pool,direct_submit,sessions}.cpp built unchanged with g++
 (AddressSanitizer + UBSan) against an emulated HSA runtime and HIP shim
 (tests/host_emu).  Emulated copy engines run their copies in order per engine
 and evaluate a dependency by polling the dependency signal's value when the
@@ -19,6 +19,8 @@ Host threads follow the kernels' device protocols:
   occupant must have polled it before the slot is handed on.
 - StagingPool sets taken and released by Queue pollers, with the fallback to
   the poller's own staging.
+- WarpSpecSession's queues (sessions.cpp): whom a destroyed session leaves
+  its queue to, and when.
 - Registered host memory mapped at another GPU address is refused as a
   copy source.
 Every landed byte is compared with the expected image, list checksums exactly.
@@ -250,3 +252,10 @@ def test_queue_batches_through_the_zero_copy_worker(poller_emu, n, t, scattered,
     out = run(poller_emu, ["queue", n, t, scattered, 2, 1], env={"GFD_ZC_WORKER": "1"})
     jobs = int(out.split("zero-copy worker jobs: ")[1].split()[0])
     assert (jobs > 0) == want_jobs, out[-2000:]
+
+
+@pytest.mark.parametrize("what", ["owner_device"])
+def test_session_queues(poller_emu, what):
+    """owner_device: a session destroyed with another device current waits for
+    its own device's kernels before its queue is left to the next session."""
+    run(os.path.join(os.path.dirname(poller_emu), "sessions_emu"), [what])
