@@ -13,7 +13,6 @@
 #include <cstring>
 #include <mutex>
 #include <thread>
-#include <vector>
 
 #include "gfd/log.h"
 #include "gfd/warp_spec_session.h"
@@ -59,7 +58,8 @@ struct SpareQueue {
     uint64_t* signals;
 };
 std::mutex g_spare_mu;
-std::vector<SpareQueue> g_spare;
+SpareQueue g_spare[WarpSpecSession::kSpareQueues];  // a fixed array: a destructor has nothing to allocate
+int g_spares = 0;
 
 // Waits until `device` is idle; the current device stays what it was.
 bool device_idle(int device) {
@@ -80,14 +80,10 @@ constexpr size_t report_offset(size_t bytes) { return (bytes + 63) & ~(size_t)63
 // ============================================================ WarpSpecSession
 
 void WarpSpecSession::release_spare_queues() {
-    std::vector<SpareQueue> all;
-    {
-        std::lock_guard<std::mutex> lock(g_spare_mu);
-        all.swap(g_spare);
-    }
-    for (const SpareQueue& q : all) {
-        gfd_hip_free(q.signals);
-        gfd_hip_host_free(q.tq);
+    std::lock_guard<std::mutex> lock(g_spare_mu);
+    for (; g_spares > 0; g_spares--) {
+        gfd_hip_free(g_spare[g_spares - 1].signals);
+        gfd_hip_host_free(g_spare[g_spares - 1].tq);
     }
 }
 
@@ -127,11 +123,11 @@ WarpSpecSession::WarpSpecSession(const WarpSpecConfig& config) : config_(config)
     gfd_hip_get_device(&device_);
     {
         std::lock_guard<std::mutex> lock(g_spare_mu);
-        for (size_t i = 0; i < g_spare.size(); i++) {
+        for (int i = 0; i < g_spares; i++) {
             if (g_spare[i].device != device_) continue;
             tq_ = g_spare[i].tq;
             d_signals_ = g_spare[i].signals;
-            g_spare.erase(g_spare.begin() + (long)i);
+            g_spare[i] = g_spare[--g_spares];
             break;
         }
     }
@@ -175,8 +171,8 @@ WarpSpecSession::~WarpSpecSession() {
     // wait for), whichever device is current here.
     if (ok_ && device_idle(device_)) {
         std::lock_guard<std::mutex> lock(g_spare_mu);
-        if (g_spare.size() < (size_t)kSpareQueues) {
-            g_spare.push_back(SpareQueue{device_, tq_, d_signals_});
+        if (g_spares < kSpareQueues) {
+            g_spare[g_spares++] = SpareQueue{device_, tq_, d_signals_};
             tq_ = nullptr;
             d_signals_ = nullptr;
         }
@@ -265,19 +261,16 @@ bool WarpSpecSession::synchronize() {
     last_elapsed_ms_ = ms_between(launch_time_, std::chrono::steady_clock::now());
     running_ = false;
     // The counters and the host-visible progress mirror (tile_chunk_done,
-    // tiled_queue.h:41): after_launch() had them written, or one copy of both.
+    // tiled_queue.h:41): after_launch() had them written, or they are copied.
     TileDeviceCounters c{};
     const uint32_t n = std::min<uint32_t>(config_.total_tiles(), (uint32_t)MAX_TILES);
     bool got = rc == 0 && reported_;
     if (got) {
         std::memcpy(&c, report_, sizeof(c));
     } else if (rc == 0) {
-        std::vector<uint64_t> w(kTileWords);
-        got = gfd_hip_memcpy_d2h(w.data(), (uint64_t)(uintptr_t)d_signals_, kTileWords * sizeof(uint64_t)) == 0;
-        if (got) {
-            std::memcpy(&c, w.data() + MAX_TILES, sizeof(c));
-            std::memcpy((void*)tq_->tile_chunk_done, w.data(), n * sizeof(uint64_t));
-        }
+        got = gfd_hip_memcpy_d2h(&c, (uint64_t)(uintptr_t)(d_signals_ + MAX_TILES), sizeof(c)) == 0 &&
+              (n == 0 || gfd_hip_memcpy_d2h((void*)tq_->tile_chunk_done, (uint64_t)(uintptr_t)d_signals_,
+                                            n * sizeof(uint64_t)) == 0);
     }
     reported_ = false;
     if (got) {

@@ -2,13 +2,25 @@
 // session leaves it to.  One scenario per run, named on the command line;
 // "pass" and status 0, or what went wrong and status 3.
 #include <cstdio>
+#include <cstdlib>
 #include <cstring>
+#include <new>
 #include <string>
 #include <vector>
 
 #include "emu.h"
 #include "gfd/hip_shim.h"
 #include "gfd/warp_spec_session.h"
+
+// Host memory runs out while this is set.
+static bool g_no_memory = false;
+void* operator new(size_t n) {
+    void* p = g_no_memory ? nullptr : std::malloc(n ? n : 1);
+    if (!p) throw std::bad_alloc();
+    return p;
+}
+void operator delete(void* p) noexcept { std::free(p); }
+void operator delete(void* p, size_t) noexcept { std::free(p); }
 
 namespace {
 
@@ -61,6 +73,31 @@ int run_owner_device() {
     return 0;
 }
 
+// A kernel that the caller launched itself, or whose read-back launch failed:
+// synchronize() copies the counters and the progress back, and the session is
+// destroyed, without host memory to allocate (both are reached from C entries,
+// where an exception would end the program).
+int run_no_memory() {
+    auto* s = new WarpSpecSession(config());
+    REQUIRE(s->ok());
+    gfd::TiledQueue* tq = s->get_launch_params().tq;
+    s->before_launch(nullptr);
+    // The kernel's writes: four tiles of 16 tokens landed.
+    for (int t = 0; t < 4; t++) tq->d_tile_chunk_done[t] = 16;
+    auto* c = reinterpret_cast<gfd::TileDeviceCounters*>(tq->d_tile_chunk_done + gfd::MAX_TILES);
+    c->next_tile = 5;
+    c->tiles_done = 4;
+    g_no_memory = true;
+    const bool done = s->synchronize();
+    g_no_memory = false;
+    REQUIRE(done && s->tiles_done() == 4 && s->error_bits() == 0 && tq->scheduler.next_tile == 4);
+    for (int t = 0; t < 5; t++) REQUIRE(tq->tile_chunk_done[t] == (t < 4 ? 16u : 0u));
+    g_no_memory = true;
+    delete s;
+    g_no_memory = false;
+    return 0;
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -68,8 +105,9 @@ int main(int argc, char** argv) {
     const std::string what = argc > 1 ? argv[1] : "";
     int rc = 4;
     if (what == "owner_device") rc = run_owner_device();
+    if (what == "no_memory") rc = run_no_memory();
     WarpSpecSession::release_spare_queues();
     if (rc == 0) std::printf("%s: pass\n", what.c_str());
-    if (rc == 4) std::fprintf(stderr, "usage: sessions_emu owner_device\n");
+    if (rc == 4) std::fprintf(stderr, "usage: sessions_emu owner_device | no_memory\n");
     return rc;
 }
