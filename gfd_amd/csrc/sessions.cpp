@@ -72,6 +72,15 @@ bool device_idle(int device) {
 }
 
 constexpr size_t kTileWords = (size_t)MAX_TILES + TILE_DEVICE_COUNTER_WORDS;
+
+// The queue's words in HBM are still the allocation that its session left:
+// hipDeviceReset() takes them away (and the queue with them).
+bool still_there(const SpareQueue& q) {
+    uint64_t base = 0, size = 0;
+    const uint64_t at = (uint64_t)(uintptr_t)q.signals, bytes = kTileWords * sizeof(uint64_t);
+    return gfd_hip_device_range(at, &base, &size) && base == at && size >= bytes && size - bytes < 4096;
+}
+
 // Where the counters' copy lies behind a pinned queue of `bytes`.
 constexpr size_t report_offset(size_t bytes) { return (bytes + 63) & ~(size_t)63; }
 
@@ -82,6 +91,7 @@ constexpr size_t report_offset(size_t bytes) { return (bytes + 63) & ~(size_t)63
 void WarpSpecSession::release_spare_queues() {
     std::lock_guard<std::mutex> lock(g_spare_mu);
     for (; g_spares > 0; g_spares--) {
+        if (!still_there(g_spare[g_spares - 1])) continue;
         gfd_hip_free(g_spare[g_spares - 1].signals);
         gfd_hip_host_free(g_spare[g_spares - 1].tq);
     }
@@ -123,12 +133,16 @@ WarpSpecSession::WarpSpecSession(const WarpSpecConfig& config) : config_(config)
     gfd_hip_get_device(&device_);
     {
         std::lock_guard<std::mutex> lock(g_spare_mu);
-        for (int i = 0; i < g_spares; i++) {
-            if (g_spare[i].device != device_) continue;
-            tq_ = g_spare[i].tq;
-            d_signals_ = g_spare[i].signals;
+        for (int i = 0; i < g_spares && !tq_;) {
+            if (g_spare[i].device != device_) {
+                i++;
+                continue;
+            }
+            if (still_there(g_spare[i])) {
+                tq_ = g_spare[i].tq;
+                d_signals_ = g_spare[i].signals;
+            }
             g_spare[i] = g_spare[--g_spares];
-            break;
         }
     }
     if (!tq_) {

@@ -159,7 +159,8 @@ public:
     // Sessions hand their queue (1 MiB of pinned host memory and its HBM
     // words) on to the next one on the device: a destroyed session leaves it,
     // with the device idle, to at most kSpareQueues spare ones, and a new one
-    // takes and clears one before it allocates.  Frees the spare ones.
+    // takes and clears one before it allocates (not one that hipDeviceReset()
+    // has taken away).  Frees the spare ones.
     static constexpr int kSpareQueues = 4;
     static void release_spare_queues();
 

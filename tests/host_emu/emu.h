@@ -50,6 +50,8 @@ void require_gpu_access(const void* p, size_t n, const char* what);
 void set_device_count(int n);
 void start_kernel(int device);
 bool kernel_runs(int device);
+// hipDeviceReset of the current device: what was allocated there is gone.
+void device_reset();
 
 // Engine stall watchdog: an engine that has polled one dependency for longer
 // than this (GFD_EMU_STALL_MS, default 5000) prints what it waits on and ends

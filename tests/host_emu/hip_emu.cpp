@@ -66,6 +66,18 @@ void note_free(void* p) {
 void set_device_count(int n) { g_devices = n; }
 void start_kernel(int device) { g_kernel[device] = true; }
 bool kernel_runs(int device) { return g_kernel[device]; }
+void device_reset() {
+    std::lock_guard<std::mutex> g(reg_mu());
+    for (auto it = reg().begin(); it != reg().end();) {
+        if (it->second.device != t_device || it->second.kind == Kind::Locked) {
+            ++it;
+            continue;
+        }
+        std::free((void*)it->first);
+        it = reg().erase(it);
+    }
+    g_kernel[t_device] = false;
+}
 
 bool find_alloc(const void* p, size_t n, Kind k, uintptr_t* base, size_t* size) {
     std::lock_guard<std::mutex> g(reg_mu());

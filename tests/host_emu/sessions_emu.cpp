@@ -98,6 +98,35 @@ int run_no_memory() {
     return 0;
 }
 
+// Sessions destroyed, then hipDeviceReset(): the queues they left are gone, and
+// sessions after it get new ones, each its own.
+int run_device_reset() {
+    emu::set_device_count(2);
+    REQUIRE(gfd_hip_set_device(1) == 0);
+    auto* other = new WarpSpecSession(config());
+    const void* kept = other->get_launch_params().tq;
+    delete other;
+    REQUIRE(gfd_hip_set_device(0) == 0);
+    {
+        WarpSpecSession a(config()), b(config()), c(config());
+        REQUIRE(a.ok() && b.ok() && c.ok());
+    }
+    emu::device_reset();
+    std::vector<WarpSpecSession*> live;
+    for (int i = 0; i < 6; i++) {
+        live.push_back(new WarpSpecSession(config()));
+        REQUIRE(live[i]->ok() && live[i]->get_launch_params().tq->scheduler.total_tiles == 4);
+        for (int j = 0; j < i; j++)
+            REQUIRE(live[i]->get_launch_params().tq != live[j]->get_launch_params().tq &&
+                    live[i]->get_launch_params().tq->d_tile_chunk_done != live[j]->get_launch_params().tq->d_tile_chunk_done);
+    }
+    for (WarpSpecSession* s : live) delete s;
+    REQUIRE(gfd_hip_set_device(1) == 0);  // the other device's queue is still there
+    WarpSpecSession d(config());
+    REQUIRE(d.ok() && d.get_launch_params().tq == kept);
+    return 0;
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -106,8 +135,9 @@ int main(int argc, char** argv) {
     int rc = 4;
     if (what == "owner_device") rc = run_owner_device();
     if (what == "no_memory") rc = run_no_memory();
+    if (what == "device_reset") rc = run_device_reset();
     WarpSpecSession::release_spare_queues();
     if (rc == 0) std::printf("%s: pass\n", what.c_str());
-    if (rc == 4) std::fprintf(stderr, "usage: sessions_emu owner_device | no_memory\n");
+    if (rc == 4) std::fprintf(stderr, "usage: sessions_emu owner_device | no_memory | device_reset\n");
     return rc;
 }
