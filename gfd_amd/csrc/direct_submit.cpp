@@ -46,15 +46,6 @@ void direct_chunk(void* p, int chunk, size_t off, size_t len) {
 }
 
 constexpr size_t kContiguousSplitMin = 8u << 20;  // split one contiguous copy above this
-// Short lists over few destination runs (at most kKernelRunEntries entries;
-// longer ones have long runs, which the copies carry well): the zero-copy
-// kernel above kKernelRuns runs or above direct_zc_min_bytes_, else a staged
-// gather with an SDMA copy per run, which starts sooner but takes 1.7 us per
-// run.  Measured on MI355X, copies against
-// kernel: 4 runs of 4 KiB 11.3 / 13.2 us, 8 of 4 KiB 18.9 / 13.1, 41 of 10 KB
-// 87.4 / 20.4, 2 of 32 KiB 12.4 / 13.2, 6 of up to 50 KB 22.1 / 16.3, 2 of 1
-// MiB 53.4 / 48.9, 60 of up to 100 KB 148 / 74.
-constexpr int kKernelRuns = 5, kKernelRunEntries = 2 * kMaxRunCopies;
 constexpr int kZcNotTaken = INT_MIN;               // direct_zero_copy: the list does not qualify
 
 }  // namespace
@@ -353,18 +344,15 @@ int CpuPollingThread::zc_launch_head(const SGEntry* entries, int k, bool uniform
 // destination.  Sources that are pinned host memory are read in place;
 // otherwise the gather pool first packs them into the (pinned) direct staging
 // and the kernel reads from there.  The entry table goes to pinned memory the
-// kernel reads.  Returns 0 or an error code.  required = false (few runs, which
-// SDMA copies can serve too): kZcNotTaken where a source is not pinned or a
-// destination is not device memory.
-int CpuPollingThread::direct_scattered(const SGEntry* entries, int count, size_t total, bool uniform, bool required) {
+// kernel reads.  Returns 0 or an error code.
+int CpuPollingThread::direct_scattered(const SGEntry* entries, int count, size_t total, bool uniform) {
     if (zc_table_cap_ < count) {
         if (zc_table_) gfd_hip_host_free(zc_table_);
         zc_table_ = nullptr;
         zc_table_cap_ = 0;
         const int cap = std::max(count, 4096);
         void* t = nullptr;
-        if (gfd_hip_host_alloc(&t, (size_t)cap * sizeof(SGEntry), GFD_HOST_DEFAULT) != 0)
-            return required ? -1 : kZcNotTaken;
+        if (gfd_hip_host_alloc(&t, (size_t)cap * sizeof(SGEntry), GFD_HOST_DEFAULT) != 0) return -1;
         zc_table_ = static_cast<SGEntry*>(t);
         zc_table_cap_ = cap;
     }
@@ -379,7 +367,6 @@ int CpuPollingThread::direct_scattered(const SGEntry* entries, int count, size_t
         if (a < dlo || b > dhi) {
             uint64_t base = 0, size = 0;
             if (!gfd_hip_device_range(a, &base, &size) || b > base + size) {
-                if (!required) return kZcNotTaken;
                 GFD_LOG_ERROR("submit_direct: destination %d is not inside a device allocation\n", i);
                 return -1;
             }
@@ -389,7 +376,6 @@ int CpuPollingThread::direct_scattered(const SGEntry* entries, int count, size_t
         if (pinned && !direct_ce_manager_.host_source_ok(entries[i].src, entries[i].size)) pinned = false;
     }
     if (!any) return 0;  // nothing to move
-    if (!required && (!pinned || !zc_ready())) return kZcNotTaken;
     bool cut = false;
     int n = count;
     if (pinned) {
@@ -565,21 +551,21 @@ double CpuPollingThread::submit_direct(const SGEntry* entries, int count) {
         }
     } else if (!dst_contig && gather_) {
         // Destinations in several runs: a packed gather with one copy per run
-        // piece, or the zero-copy kernel when there are many runs.
+        // piece, or the zero-copy kernel when there are many runs.  Short lists
+        // of few runs stay on the copies although the kernel is faster (copies
+        // against kernel: 8 runs of 4 KiB 18.9 / 13.1 us, 41 of 10 KB 87 / 20,
+        // 60 of up to 100 KB 148 / 74): their callers never needed a free
+        // compute unit or hardware queue, and a kernel launched here waits
+        // behind one of theirs that spins until this list has landed.
         const int nr = dst_runs(entries, count, kMaxRunCopies, direct_runs_);
-        if (nr <= kMaxRunCopies && count <= kKernelRunEntries &&
-            (nr > kKernelRuns || total > direct_zc_min_bytes_) && total <= direct_zc_max_bytes_ && zc_pinned != 0 &&
-            (err = direct_scattered(entries, count, total, uniform, false)) != kZcNotTaken) {
-            // done by the zero-copy kernel (err 0) or failed
-        } else if (nr <= kMaxRunCopies && direct_staging_ && total <= direct_staging_size_) {
-            err = 0;
+        if (nr <= kMaxRunCopies && direct_staging_ && total <= direct_staging_size_) {
             std::lock_guard<std::mutex> lock(gather_mutex_);
             RunCopyCtx ctx{this, &direct_ce_manager_, direct_staging_, direct_runs_.data(), nr, 0, nch, 0, 0};
             gather_->run(entries, count, total, direct_staging_, direct_chunk_bytes_, run_copy_chunk, &ctx,
                          uniform ? 1 : 0);
             err = ctx.err;
         } else if (nr > kMaxRunCopies) {
-            err = direct_scattered(entries, count, total, uniform, true);
+            err = direct_scattered(entries, count, total, uniform);
         } else {
             err = direct_ce_manager_.submit_scatter_gather(entries, count);
         }

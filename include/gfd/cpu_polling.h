@@ -255,7 +255,7 @@ private:
     // uniform_hint as for GatherEngine::run.
     bool gather_through_staging(const SGEntry* e, int count, size_t total, const DstRun* runs = nullptr,
                                 int nruns = 0, int uniform_hint = -1);
-    int direct_scattered(const SGEntry* entries, int count, size_t total, bool uniform, bool required);
+    int direct_scattered(const SGEntry* entries, int count, size_t total, bool uniform);
     int direct_zero_copy(const SGEntry* entries, int count, size_t total, bool uniform, bool sources_checked);
     int direct_worker(const SGEntry* entries, int count, size_t total);
     bool queue_worker_copy(const SGEntry* e, int count, size_t total);

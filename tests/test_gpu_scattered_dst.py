@@ -85,8 +85,11 @@ def blocks_layout(n, t, nblocks, gap):
     return offs, nblocks * (per * t + gap)
 
 
-# Either side of the lines between the SDMA copies and the kernel: 5 runs, 64
-# KiB, 64 runs, 8 MiB; pageable sources stay on the copies.
+TRACE_ZC_LAUNCH = 14
+
+
+# Either side of the line between the SDMA copies (up to 64 runs, no kernel)
+# and the kernel, with either side of 64 KiB and of 8 MiB, which do not move it.
 @pytest.mark.parametrize("n,t,nblocks", [(4, 4096, 4), (5, 4096, 5), (6, 4096, 6), (2, 32768, 2), (2, 32784, 2),
                                          (16, 1000, 16), (41, 10169, 41), (64, 100, 64), (65, 100, 65),
                                          (8, 1 << 20, 8), (9, 1 << 20, 9), (700, 900, 7)])
@@ -95,10 +98,17 @@ def test_direct_short_lists_of_runs(direct_poller, n, t, nblocks, pageable):
     log("direct short runs n=%d t=%d blocks=%d pageable=%d" % (n, t, nblocks, pageable))
     offs, region = blocks_layout(n, t, nblocks, 48)
     c = Case(n, t, offs, region, pageable)
-    for _ in range(2):
-        c.dst.fill(SENTINEL)
-        assert direct_poller.submit_direct(c.entries, n) > 0
-        c.check()
+    direct_poller.set_trace(True)
+    try:
+        for _ in range(2):
+            c.dst.fill(SENTINEL)
+            direct_poller.read_trace()
+            assert direct_poller.submit_direct(c.entries, n) > 0
+            kinds = direct_poller.read_trace()["kind"]
+            assert int((kinds == TRACE_ZC_LAUNCH).sum()) == (1 if nblocks > 64 else 0)
+            c.check()
+    finally:
+        direct_poller.set_trace(False)
 
 
 @pytest.mark.parametrize("n,t,nblocks", [(4096, 4096, 10), (2048, 1000, 64), (300, 4096, 2), (8192, 4096, 40)])

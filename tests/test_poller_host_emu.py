@@ -120,6 +120,16 @@ def test_ragged_entries_over_destination_runs(poller_emu, path, nruns):
         assert zero_copy_launches(out) == [1 if nruns == 1 else 0] * 2, out[-2000:]
 
 
+@pytest.mark.parametrize("n,nruns,launches", [(2, 2, 0), (8, 8, 0), (41, 41, 0), (64, 64, 0), (128, 40, 0),
+                                              (65, 65, 1), (200, 100, 1)])
+def test_direct_short_lists_of_runs_need_no_kernel(poller_emu, n, nruns, launches):
+    # Up to 64 destination runs are copied by the engines whatever their
+    # number and size: a caller's kernel that spins until such a list has
+    # landed may hold the hardware queue that a kernel would be launched on.
+    out = run(poller_emu, ["ragged", "direct", n, nruns, 2, 3], env={"GFD_EMU_MAX_ENTRY": "20000"})
+    assert zero_copy_launches(out) == [launches] * 2, out[-2000:]
+
+
 @pytest.mark.parametrize("n,max_entry", [(5, 200000), (40, 70000), (63, 9000), (3, 100000)])
 def test_direct_short_ragged_list_cut_into_pieces(poller_emu, n, max_entry):
     # A short destination-contiguous list of large ragged entries: the
