@@ -67,14 +67,14 @@ __device__ __forceinline__ int row_min(int v) {
 }
 
 // The lowest expert that holds the largest of the token's logits, in every
-// lane.  A NaN is never the largest; 0 if all are NaN.
-__device__ __forceinline__ int argmax16(const float (&x)[kTokExperts], int num_experts, int lane) {
+// lane.  A NaN ranks behind everything; `none` if all are NaN.
+__device__ __forceinline__ int argmax16(const float (&x)[kTokExperts], int num_experts, int lane, int none) {
     const float top = row_max(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])));
     int i = 64;
 #pragma unroll
     for (int k = kTokExperts - 1; k >= 0; k--) i = x[k] == top ? lane + k * kTokLanes : i;
     i = row_min(i);
-    return i < num_experts ? i : 0;
+    return i < num_experts ? i : none;
 }
 
 typedef int int2v __attribute__((ext_vector_type(2), aligned(4)));
@@ -92,13 +92,16 @@ __device__ __forceinline__ void load_logits(float (&x)[kTokExperts], const float
     }
 }
 
-// The token's two experts, in all of its lanes.
+// The token's two experts, in all of its lanes: always two, since the lists
+// hold a row per choice.  The first leaves the second pass as a NaN, which no
+// logit ties with (-inf may be the largest that is left); where only NaNs are
+// left, the lowest other expert is taken.
 __device__ __forceinline__ int2v top2_of(float (&x)[kTokExperts], int num_experts, int lane) {
-    const int first = argmax16(x, num_experts, lane);
+    const int first = argmax16(x, num_experts, lane, 0);
 #pragma unroll
     for (int k = 0; k < kTokExperts; k++)
-        if (lane + k * kTokLanes == first) x[k] = -INFINITY;
-    return int2v{first, argmax16(x, num_experts, lane)};
+        if (lane + k * kTokLanes == first) x[k] = __builtin_nanf("");
+    return int2v{first, argmax16(x, num_experts, lane, first == 0 ? 1 : 0)};
 }
 
 // Latency bound: 4 loads, then two chains of 8 cross-lane steps.  16 tokens

@@ -243,7 +243,7 @@ int gfd_zero_copy_scatter_tokens(const uint64_t* dst_addrs, const void* src, uin
  * warp-specialised path, reference include/gfd/sg_warp_spec.cuh and
  * examples/09_sg_warp_spec.cu, kept entirely on the GPU) ---- */
 /* Top-2 experts per token of logits[num_tokens][num_experts] (fp32, HBM;
- * ties -> lower expert id) into top2[2*num_tokens]; per-expert row lists in
+ * ties -> lower expert id, NaN behind everything, always two experts) into top2[2*num_tokens]; per-expert row lists in
  * token order: offsets[num_experts+1], row_token[2*num_tokens] (expert-major). */
 int gfd_moe_route(const float* logits, int num_tokens, int num_experts, int* top2, int* offsets,
                   int* row_token, void* stream);

@@ -174,3 +174,36 @@ def test_route_of_nan_rows_stays_in_range(T):
     assert o[0] == 0 and o[E] == 2 * T and (np.diff(o) >= 0).all()
     r = rows.download().view(np.int32)
     assert (r >= 0).all() and (r < T).all()
+
+
+@pytest.mark.parametrize("T", [300, 5000])
+@pytest.mark.parametrize("E", [2, 5, 64])
+def test_route_of_rows_without_two_finite_logits(T, E):
+    """Rows of NaN, -inf and +inf: the two experts are distinct, so that every
+    row of the lists is written; a NaN ranks behind everything, ties go to the
+    lower expert."""
+    print("route of NaN and infinite rows T=%d E=%d" % (T, E), flush=True)
+    rng = np.random.default_rng(T + E)
+    logits = rng.standard_normal((T, E), dtype=np.float32)
+    logits[rng.random((T, E)) < 0.4] = np.nan
+    one = rng.integers(0, E, T)
+    for kind, (fill, at) in enumerate([(np.nan, None), (np.nan, 1.0), (-np.inf, None), (-np.inf, 1.0), (np.nan, -np.inf),
+                                       (-np.inf, np.nan), (np.inf, np.nan), (-np.inf, np.inf), (np.inf, None)]):
+        t = np.arange(kind, T, 12)
+        logits[t] = fill
+        if at is not None:
+            logits[t, np.where(t % 24 == kind, one[t], 0)] = at  # at any expert, and at expert 0
+    top2 = oracle.moe_top2(logits)
+    offsets, rows = oracle.moe_lists(top2, E)
+    d = gfd_amd.DeviceBuffer(logits.nbytes)
+    d.upload(logits)
+    outs = [gfd_amd.DeviceBuffer(4 * n) for n in (2 * T, E + 1, 2 * T)]
+    for o in outs:
+        o.fill(0xCD)
+    gfd_amd.moe_route(d.ptr, T, E, outs[0].ptr, outs[1].ptr, outs[2].ptr)
+    gfd_amd.synchronize()
+    got = [o.download().view(np.int32) for o in outs]
+    assert (top2[:, 0] != top2[:, 1]).all()
+    assert (got[0] == top2.reshape(-1)).all()
+    assert (got[1] == offsets).all()
+    assert (got[2] == rows).all()
