@@ -50,18 +50,18 @@ constexpr int kZcNotTaken = INT_MIN;               // direct_zero_copy: the list
 
 }  // namespace
 
-// The zero-copy SG kernel (and the zero-copy worker) gives each entry of a
-// short list a wave of its own, so a list of fewer entries than its `waves`
-// waves leaves waves idle while a few stream whole large entries.  Such a
-// list's entries are cut into pieces of at least 4 KiB, a multiple of 16
-// bytes each (an entry's last piece takes what is left), so the pieces keep
-// each entry's alignment.  The piece size is set for waves - count waves,
-// since each entry's last piece may be a short one: the table then has at
-// most `waves` records, one per wave (*presliced = true; the kernel's
-// presliced launch does not cut them again).  Writes the table to out (at
-// most cap records) and returns its length, or copies the entries unchanged
-// (*presliced = false) when the list is long enough or the pieces would not
-// fit.  The caller guarantees count <= cap.
+// The zero-copy worker gives each entry of a short list a wave of its own, and
+// the zero-copy SG kernel cuts entries by their number without knowing their
+// sizes, so a list of fewer entries than its `waves` waves leaves waves idle
+// while a few stream whole large entries.  Such a list's entries are cut here
+// into pieces of at least 4 KiB, a multiple of 16 bytes each (an entry's last
+// piece takes what is left), so the pieces keep each entry's alignment.  The
+// piece size is set for waves - count waves, since each entry's last piece may
+// be a short one: the table then has at most `waves` records, one per wave
+// (*presliced = true; the kernel's presliced launch does not cut them again).
+// Writes the table to out (at most cap records) and returns its length, or
+// copies the entries unchanged (*presliced = false) when the list is long
+// enough or the pieces would not fit.  The caller guarantees count <= cap.
 int zc_fill_sg_table(const SGEntry* in, int count, size_t total, SGEntry* out, int cap, bool* presliced, int waves) {
     constexpr size_t kMinPiece = 4096;
     *presliced = false;
@@ -93,8 +93,16 @@ int zc_fill_sg_table(const SGEntry* in, int count, size_t total, SGEntry* out, i
 // pieces would be large, and the waves unequal).  Measured on MI355X, 64
 // against 128: 40 entries of up to 20 KB 22.8 -> 21.8 us, 60 of up to 30 KB
 // 32.0 -> 30.2, 40 of up to 100 KB 56.1 -> 53.5; but 20 of up to 40 KB 21.0
-// -> 21.6.
-static int cut_waves(int count, int waves) { return 3 * (int64_t)count > waves ? 2 * waves : waves; }
+// -> 21.6.  An explicit GFD_ZC_WAVES is the number of waves launched, so there
+// are no more pieces than that.
+static int cut_waves(int count) {
+    static const int waves = gfd_zero_copy_target_waves();
+    static const bool fixed = [] {
+        const char* v = std::getenv("GFD_ZC_WAVES");
+        return v && *v;
+    }();
+    return !fixed && 3 * (int64_t)count > waves ? 2 * waves : waves;
+}
 
 void run_copy_chunk(void* p, int chunk, size_t off, size_t len) {
     RunCopyCtx* c = (RunCopyCtx*)p;
@@ -263,8 +271,7 @@ int CpuPollingThread::direct_zero_copy(const SGEntry* entries, int count, size_t
             zc_table_cap_ = cap;
         }
         bool cut = false;
-        static const int kWaves = gfd_zero_copy_target_waves();
-        const int n = zc_fill_sg_table(entries, count, total, zc_table_, zc_table_cap_, &cut, cut_waves(count, kWaves));
+        const int n = zc_fill_sg_table(entries, count, total, zc_table_, zc_table_cap_, &cut, cut_waves(count));
         rc = (cut ? gfd_zero_copy_gather_signal_presliced : gfd_zero_copy_gather_signal)(
             reinterpret_cast<const gfd_sg_entry*>(zc_table_), n, zc_counter_, zc_done_, gen, zc_stream_);
     }
@@ -328,8 +335,7 @@ int CpuPollingThread::zc_launch_head(const SGEntry* entries, int k, bool uniform
         size_t bytes = 0;
         for (int i = 0; i < k; i++) bytes += entries[i].size;
         bool cut = false;
-        static const int kWaves = gfd_zero_copy_target_waves();
-        const int n = zc_fill_sg_table(entries, k, bytes, zc_table_, zc_table_cap_, &cut, cut_waves(k, kWaves));
+        const int n = zc_fill_sg_table(entries, k, bytes, zc_table_, zc_table_cap_, &cut, cut_waves(k));
         rc = (cut ? gfd_zero_copy_gather_signal_presliced : gfd_zero_copy_gather_signal)(
             reinterpret_cast<const gfd_sg_entry*>(zc_table_), n, zc_counter_, zc_done_, g, zc_stream_);
     }
@@ -379,8 +385,7 @@ int CpuPollingThread::direct_scattered(const SGEntry* entries, int count, size_t
     bool cut = false;
     int n = count;
     if (pinned) {
-        static const int kWaves = gfd_zero_copy_target_waves();
-        n = zc_fill_sg_table(entries, count, total, zc_table_, zc_table_cap_, &cut, cut_waves(count, kWaves));
+        n = zc_fill_sg_table(entries, count, total, zc_table_, zc_table_cap_, &cut, cut_waves(count));
     } else {
         if (!direct_staging_ || total > direct_staging_size_ || !gather_) return -1;
         {

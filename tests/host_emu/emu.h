@@ -38,6 +38,8 @@ uintptr_t locked_agent_base(uintptr_t base);
 // Launches of the emulated zero-copy kernels (the Direct path's kernel
 // route), so a scenario can tell which route a call took.
 unsigned zero_copy_launches();
+// Records in the table of the last entry-list launch.
+int zero_copy_records();
 
 // Aborts the process, as a GPU page fault would end it, unless [p, p + n) is
 // pinned host memory or device memory (n = 0 passes).

@@ -109,6 +109,7 @@ int g_handle = 0;
 
 namespace {
 std::atomic<unsigned> g_zc_launches{0};
+std::atomic<int> g_zc_records{0};
 
 void require_gpu_readable(const void* p, size_t n, const char* what) { emu::require_gpu_access(p, n, what); }
 }
@@ -128,6 +129,7 @@ void require_gpu_access(const void* p, size_t n, const char* what) {
 }  // namespace emu
 namespace emu {
 unsigned zero_copy_launches() { return g_zc_launches.load(); }
+int zero_copy_records() { return g_zc_records.load(); }
 }  // namespace emu
 
 extern "C" {
@@ -286,6 +288,7 @@ int gfd_zero_copy_gather_signal(const gfd_sg_entry* entries, int count, unsigned
                                 uint64_t* done_word, uint64_t done_value, void*) {
     if (!done_counter || !done_word || count < 0 || (count > 0 && !entries)) return 1;
     g_zc_launches++;
+    g_zc_records = count;
     for (int i = 0; i < count; i++)
         require_gpu_readable((const void*)(uintptr_t)entries[i].src, entries[i].size, "zc_gather_sg");
     for (int i = 0; i < count; i++)
@@ -300,6 +303,9 @@ int gfd_zero_copy_gather_signal_presliced(const gfd_sg_entry* entries, int count
     return gfd_zero_copy_gather_signal(entries, count, done_counter, done_word, done_value, stream);
 }
 
-int gfd_zero_copy_target_waves(void) { return 64; }
+int gfd_zero_copy_target_waves(void) {
+    const char* v = std::getenv("GFD_ZC_WAVES");
+    return v && *v ? std::atoi(v) : 64;
+}
 
 }  // extern "C"

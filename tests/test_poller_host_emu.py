@@ -140,6 +140,20 @@ def test_direct_short_ragged_list_cut_into_pieces(poller_emu, n, max_entry):
     assert zero_copy_launches(out) == [1] * 2, out[-2000:]
 
 
+@pytest.mark.parametrize("waves,least,most", [(None, 65, 128), (64, 41, 64), (100, 41, 100)])
+def test_direct_short_list_cut_for_the_waves_that_are_launched(poller_emu, waves, least, most):
+    # 40 large entries are cut for twice the default 64 waves; an explicit
+    # GFD_ZC_WAVES is the number launched, and then the most pieces there are
+    # (a piece is one wave's work).
+    env = {"GFD_EMU_MAX_ENTRY": "70000"}
+    if waves:
+        env["GFD_ZC_WAVES"] = str(waves)
+    out = run(poller_emu, ["ragged", "direct", 40, 1, 2, 5], env=env)
+    assert zero_copy_launches(out) == [1] * 2, out[-2000:]
+    records = [int(l.split(":")[1]) for l in out.splitlines() if l.startswith("zero-copy records:")]
+    assert all(least <= r <= most for r in records) and len(records) == 2, records
+
+
 @pytest.mark.parametrize("zc_min,launches", [(0, 1), (64 << 20, 0)])
 def test_direct_zero_copy_minimum(poller_emu, zc_min, launches):
     # The one-run list of about 3 MiB: on the zero-copy route with no minimum,
