@@ -79,6 +79,44 @@ def test_moe_through_session(T, E, dim, rpl, blocks, cw):
         sess.close()
 
 
+@pytest.mark.parametrize("dim,rpl", [(512, 64), (512, 15), (1024, 9), (1536, 13), (2048, 4), (2560, 5), (3072, 2)])
+def test_moe_session_to_host_rows(dim, rpl):
+    """Rows staged on their way from HBM to pinned host memory (evicted and
+    normalised at once): groups of 14, 7, 4, 3 and 2 rows and single ones,
+    with groups cut short at the ends of the lists.  Rows byte-exact, the
+    RMSNorm within one bf16 ulp, and bytes behind both outputs untouched."""
+    T, E, cw = 230, 6, 3
+    print("moe session to host rows dim=%d rows/list=%d" % (dim, rpl), flush=True)
+    m = Moe(T, E, dim)
+    m.route()
+    n, nbytes = 2 * T, 2 * T * m.row_bytes
+    rows = m.expected_rows()
+    ref = oracle.rmsnorm_rows(oracle.bf16_to_f32(rows), oracle.bf16_to_f32(m.weight), 1e-6)
+    src = gfd_amd.DeviceBuffer(m.host.nbytes)
+    src.upload(m.host.array)
+    dst = gfd_amd.HostBuffer(nbytes + 256)
+    sess = gfd_amd.SGWarpSpecSession(num_compute_warps=cw, num_blocks=4, idle_limit_ms=10000)
+    try:
+        for _ in range(2):
+            dst.array[:] = 0xCD
+            m.d_out.fill(0xCD)
+            sess.reset()
+            sess.launch_moe(src.ptr, m.stride, m.T, m.d_offsets.ptr, m.d_rows.ptr, m.E, n, m.row_bytes, dst.ptr,
+                            m.d_out.ptr, m.d_weight.ptr, 1e-6, rpl)
+            gfd_amd.synchronize()
+            sess.synchronize(0)
+            st = sess.stats()
+            assert st["error_bits"] == 0 and st["units_done"] == n and st["bytes"] == nbytes
+            assert (dst.array[:nbytes].view(np.uint16).reshape(n, dim) == rows).all()
+            assert (dst.array[nbytes:] == 0xCD).all()
+            out = m.d_out.download()
+            y = oracle.bf16_to_f32(out[:nbytes].view(np.uint16).reshape(n, dim))
+            assert np.all(np.abs(y - ref) <= np.abs(ref) * 2.0 ** -7 + 1e-6)
+            assert (out[nbytes:] == 0xCD).all()
+    finally:
+        sess.close()
+
+
 def test_moe_session_with_host_lists_queued_before_launch():
     """Host lists queued before launch_moe land in the same launch, and the
     session's lists_done counts them: the GPU submitter must wait for those
