@@ -84,7 +84,10 @@ struct TokenRmsSinT {
     // hand a chunk's tokens to several compute waves in groups.
     static constexpr bool kSplitsChunks = true;
 
-    __device__ void operator()(ChunkView c) const {
+    // Inlined at both of its call sites: as a call it needs a frame of 112
+    // bytes of scratch per lane and 120 VGPRs instead of 112 (96 bytes and 167
+    // instead of 139 in the 9-wave kernel), at the same speed (within 0.6%).
+    [[clang::always_inline]] __device__ void operator()(ChunkView c) const {
         const uint32_t nf = c.token_size / 4;
         const uint32_t lane = (uint32_t)c.lane_id;
         if (((uintptr_t)c.base_ptr & 15) == 0 && (c.token_size & 15) == 0 && nf >= 4 && nf / 4 <= 64u * kRegVecs) {
