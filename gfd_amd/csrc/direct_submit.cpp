@@ -104,6 +104,26 @@ static int cut_waves(int count) {
     return !fixed && 3 * (int64_t)count > waves ? 2 * waves : waves;
 }
 
+// Launches the kernel over the n records of a table that zc_fill_sg_table
+// wrote.  The host knows here what the kernel does not, and the table lies in
+// pinned memory, so the kernel's own slices, whose strided order has every
+// wave read records all over it, only serve a few uncut entries.  Measured on
+// MI355X, submit_direct into scattered pages, slices / whole entries on 64
+// waves / a wave each:
+//   200 x 4 KiB 29.9 / 27.4 / 29.2 us, 256 x 4 KiB 32.3 / 31.7 / 35.4,
+//   512 x 2 KiB 33.1 / 32.9 / 35.7;
+//   100 of up to 4 KB 18.1 / 18.0 / 16.8, 128 of up to 8 KB 24.9 / 24.6 / 23.4,
+//   256 of up to 16 KB 53.7 / 57.0 / 52.6, 512 of up to 40 KB 207.9 / 215 / 207.5.
+static int zc_launch_table(const SGEntry* table, int n, bool cut, bool uniform, unsigned int* counter, uint64_t* done,
+                           uint64_t gen, gfd_stream_t stream) {
+    constexpr int kFew = 32, kSpread = 512;
+    const auto* t = reinterpret_cast<const gfd_sg_entry*>(table);
+    if (cut || (!uniform && n > kFew && n <= kSpread))
+        return gfd_zero_copy_gather_signal_presliced(t, n, counter, done, gen, stream);
+    if (n > kFew) return gfd_zero_copy_gather_signal_equal(t, n, counter, done, gen, stream);
+    return gfd_zero_copy_gather_signal(t, n, counter, done, gen, stream);
+}
+
 void run_copy_chunk(void* p, int chunk, size_t off, size_t len) {
     RunCopyCtx* c = (RunCopyCtx*)p;
     const size_t end = off + len;
@@ -272,8 +292,7 @@ int CpuPollingThread::direct_zero_copy(const SGEntry* entries, int count, size_t
         }
         bool cut = false;
         const int n = zc_fill_sg_table(entries, count, total, zc_table_, zc_table_cap_, &cut, cut_waves(count));
-        rc = (cut ? gfd_zero_copy_gather_signal_presliced : gfd_zero_copy_gather_signal)(
-            reinterpret_cast<const gfd_sg_entry*>(zc_table_), n, zc_counter_, zc_done_, gen, zc_stream_);
+        rc = zc_launch_table(zc_table_, n, cut, uniform, zc_counter_, zc_done_, gen, zc_stream_);
     }
     if (rc != 0) return rc;
     trace(TRACE_ZC_LAUNCH, (uint32_t)count, total);
@@ -336,8 +355,7 @@ int CpuPollingThread::zc_launch_head(const SGEntry* entries, int k, bool uniform
         for (int i = 0; i < k; i++) bytes += entries[i].size;
         bool cut = false;
         const int n = zc_fill_sg_table(entries, k, bytes, zc_table_, zc_table_cap_, &cut, cut_waves(k));
-        rc = (cut ? gfd_zero_copy_gather_signal_presliced : gfd_zero_copy_gather_signal)(
-            reinterpret_cast<const gfd_sg_entry*>(zc_table_), n, zc_counter_, zc_done_, g, zc_stream_);
+        rc = zc_launch_table(zc_table_, n, cut, uniform, zc_counter_, zc_done_, g, zc_stream_);
     }
     if (rc != 0) return rc;
     trace(TRACE_ZC_LAUNCH, (uint32_t)k, 0);
@@ -401,8 +419,7 @@ int CpuPollingThread::direct_scattered(const SGEntry* entries, int count, size_t
     }
     if (!zc_ready()) return -1;
     const uint64_t gen = ++zc_gen_;
-    int rc = (cut ? gfd_zero_copy_gather_signal_presliced : gfd_zero_copy_gather_signal)(
-        reinterpret_cast<const gfd_sg_entry*>(zc_table_), n, zc_counter_, zc_done_, gen, zc_stream_);
+    int rc = zc_launch_table(zc_table_, n, cut, uniform, zc_counter_, zc_done_, gen, zc_stream_);
     if (rc != 0) return rc;
     trace(TRACE_ZC_LAUNCH, (uint32_t)count, total);
     rc = zc_wait(gen);

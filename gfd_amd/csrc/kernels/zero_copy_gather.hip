@@ -32,6 +32,7 @@
 #include <cstdint>
 #include <cstdlib>
 
+#include "gfd/hip_shim.h"
 #include "gfd/wave_ops.h"
 
 #include "gfd_capi.h"
@@ -55,8 +56,10 @@ constexpr int kDefaultLds = 0;
 // 512 KiB (16-64): 500 x 3333 B 46.4 -> 35.0 us, 2048 x 2 KiB 85.6 -> 79.7, 2 x
 // 1 MiB 48.3 -> 41.1, 2048 x 512 B 23.8 -> 22.2, 4096 x 3000 B 237 -> 233;
 // 8192 x 4 KiB the same (607).  Larger jobs keep 64 waves (2048 x 64 KiB 2414
-// us, 2419 with 128), and 256 lose 1% from 32 MiB on.  With a completion
-// signal every workgroup writes its L2 back: there the old 16-64 stand.
+// us, 2419 with 128), and 256 lose 1% from 32 MiB on.  Jobs with a completion
+// signal still take one wave per 512 KiB, 16-64 (128 waves would gain there as
+// well: 500 x 3333 B 52.1 -> 40.8 us, 2 x 1 MiB 54.2 -> 47.2, 2048 x 2 KiB 91.5
+// -> 85.6, 4096 x 3000 B 242.7 -> 239.8, 8192 x 4 KiB the same).
 constexpr uint64_t kScatterBytesPerWave = 512 * 1024, kScatterWideBytes = 32ull << 20;
 constexpr int kScatterMinWaves = 16, kScatterMaxWaves = 64, kScatterWideWaves = 128;
 constexpr int kScatterUnroll = 8;
@@ -294,15 +297,23 @@ int short_list_waves() { return std::max(4, env_int(kGatherShape.waves_env, kGat
 constexpr int kSgUnits = 1024, kShortSg = 32;
 constexpr ShapeDefaults kSgShape{kBytesPerWave, kMaxWaves, kMaxWaves, kDefaultUnroll, "GFD_ZC_WAVES", "GFD_ZC_UNROLL"};
 
-// slice: the table is the caller's list as it is.  Without it, each record is
-// one wave's work (the caller has cut the list into pieces already), up to
-// kMaxWaves of them.
-int launch_gather_sg(const gfd_sg_entry* entries, int count, void* stream, GridDone done, bool slice = true) {
+// What the host knows of a list's entries, and so how the waves take them.
+enum class Entries {
+    kUnknown,  // the table is the caller's list as it is: slices, as above
+    kEqual,    // whole, a run of them to each of 64 waves
+    kSpread,   // whole, a wave each up to kMaxWaves (pieces, or unequal entries)
+};
+
+int launch_gather_sg(const gfd_sg_entry* entries, int count, void* stream, GridDone done,
+                     Entries kind = Entries::kUnknown) {
     if (count < 0 || (count > 0 && !entries)) return (int)hipErrorInvalidValue;
     if (count == 0) return 0;
-    const uint32_t pieces = slice && 2 * (int64_t)count <= kSgUnits ? (uint32_t)(kSgUnits / count) : 1u;
+    const uint32_t pieces =
+        kind == Entries::kUnknown && 2 * (int64_t)count <= kSgUnits ? (uint32_t)(kSgUnits / count) : 1u;
+    const bool few_waves = kind == Entries::kEqual ||
+                           (kind == Entries::kUnknown && (done.host_word || count <= kShortSg));
     const Shape s = shape_for((uint64_t)count * pieces, (uint64_t)count * pieces * 4096,
-                              slice && (done.host_word || count <= kShortSg) ? kGatherShape : kSgShape);
+                              few_waves ? kGatherShape : kSgShape);
     if (s.lds)
         hipLaunchKernelGGL(zc_gather_sg<true>, dim3(s.blocks), dim3(kBlock), 0, (hipStream_t)stream, entries,
                            (uint32_t)count, pieces, s.per_wave, s.unroll, done);
@@ -356,7 +367,14 @@ extern "C" int gfd_zero_copy_gather_signal_presliced(const gfd_sg_entry* entries
                                                      unsigned int* done_counter, uint64_t* done_word,
                                                      uint64_t done_value, void* stream) {
     if (!done_counter || !done_word) return (int)hipErrorInvalidValue;
-    return launch_gather_sg(entries, count, stream, grid_done(done_counter, done_word, done_value), false);
+    return launch_gather_sg(entries, count, stream, grid_done(done_counter, done_word, done_value), Entries::kSpread);
+}
+
+extern "C" int gfd_zero_copy_gather_signal_equal(const void* entries, int count, unsigned int* done_counter,
+                                                 uint64_t* done_word, uint64_t done_value, void* stream) {
+    if (!done_counter || !done_word) return (int)hipErrorInvalidValue;
+    return launch_gather_sg(static_cast<const gfd_sg_entry*>(entries), count, stream,
+                            grid_done(done_counter, done_word, done_value), Entries::kEqual);
 }
 
 extern "C" int gfd_zero_copy_target_waves(void) { return short_list_waves(); }

@@ -74,6 +74,10 @@ int gfd_ws_prepare_launch(uint64_t* d, uint64_t words, gfd_stream_t stream);
 // the stream is synchronised.
 int gfd_session_report(const uint64_t* src0, uint64_t* dst0, uint64_t n0, const uint64_t* src1, uint64_t* dst1,
                        uint64_t n1, gfd_stream_t stream);
+// gfd_zero_copy_gather_signal for entries the caller knows to be of one size:
+// whole entries, a run of them to each of 64 waves.
+int gfd_zero_copy_gather_signal_equal(const void* entries, int count, unsigned int* done_counter, uint64_t* done_word,
+                                      uint64_t done_value, void* stream);
 }
 
 extern "C" {

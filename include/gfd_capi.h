@@ -213,10 +213,10 @@ int gfd_zero_copy_scatter_tokens_signal(const uint64_t* dst_addrs, const void* s
 int gfd_zero_copy_gather_signal(const gfd_sg_entry* entries, int count, unsigned int* done_counter,
                                 uint64_t* done_word, uint64_t done_value, void* stream);
 /* gfd_zero_copy_gather_signal for a table the caller has already cut into
- * pieces (no reference counterpart; used by submit_direct, whose
- * zc_fill_sg_table cuts a short list of large entries by size): the kernel
- * does not slice the entries again by count, so each record stays one wave's
- * work. */
+ * pieces, or whose entries are not to be cut (no reference counterpart; used
+ * by submit_direct, whose zc_fill_sg_table cuts a short list of large entries
+ * by size): the kernel does not slice the entries by count, so each record
+ * stays one wave's work, on up to 256 waves. */
 int gfd_zero_copy_gather_signal_presliced(const gfd_sg_entry* entries, int count, unsigned int* done_counter,
                                           uint64_t* done_word, uint64_t done_value, void* stream);
 /* Waves the zero-copy gather kernels give a short list (no reference
@@ -243,8 +243,9 @@ int gfd_zero_copy_scatter_tokens(const uint64_t* dst_addrs, const void* src, uin
  * warp-specialised path, reference include/gfd/sg_warp_spec.cuh and
  * examples/09_sg_warp_spec.cu, kept entirely on the GPU) ---- */
 /* Top-2 experts per token of logits[num_tokens][num_experts] (fp32, HBM;
- * ties -> lower expert id, NaN behind everything, always two experts) into top2[2*num_tokens]; per-expert row lists in
- * token order: offsets[num_experts+1], row_token[2*num_tokens] (expert-major). */
+ * ties -> lower expert id, NaN behind everything, always two experts) into
+ * top2[2*num_tokens]; per-expert row lists in token order:
+ * offsets[num_experts+1], row_token[2*num_tokens] (expert-major). */
 int gfd_moe_route(const float* logits, int num_tokens, int num_experts, int* top2, int* offsets,
                   int* row_token, void* stream);
 /* gfd_moe_route for callers that cannot allocate (code under HIP graph

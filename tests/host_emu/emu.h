@@ -40,6 +40,8 @@ uintptr_t locked_agent_base(uintptr_t base);
 unsigned zero_copy_launches();
 // Records in the table of the last entry-list launch.
 int zero_copy_records();
+// How it was launched: "sliced" (by the kernel), "presliced" (a wave each) or "equal".
+const char* zero_copy_kind();
 
 // Aborts the process, as a GPU page fault would end it, unless [p, p + n) is
 // pinned host memory or device memory (n = 0 passes).

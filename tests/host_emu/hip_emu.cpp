@@ -110,6 +110,7 @@ int g_handle = 0;
 namespace {
 std::atomic<unsigned> g_zc_launches{0};
 std::atomic<int> g_zc_records{0};
+std::atomic<const char*> g_zc_kind{""};
 
 void require_gpu_readable(const void* p, size_t n, const char* what) { emu::require_gpu_access(p, n, what); }
 }
@@ -130,6 +131,7 @@ void require_gpu_access(const void* p, size_t n, const char* what) {
 namespace emu {
 unsigned zero_copy_launches() { return g_zc_launches.load(); }
 int zero_copy_records() { return g_zc_records.load(); }
+const char* zero_copy_kind() { return g_zc_kind.load(); }
 }  // namespace emu
 
 extern "C" {
@@ -289,6 +291,7 @@ int gfd_zero_copy_gather_signal(const gfd_sg_entry* entries, int count, unsigned
     if (!done_counter || !done_word || count < 0 || (count > 0 && !entries)) return 1;
     g_zc_launches++;
     g_zc_records = count;
+    g_zc_kind = "sliced";
     for (int i = 0; i < count; i++)
         require_gpu_readable((const void*)(uintptr_t)entries[i].src, entries[i].size, "zc_gather_sg");
     for (int i = 0; i < count; i++)
@@ -300,7 +303,17 @@ int gfd_zero_copy_gather_signal(const gfd_sg_entry* entries, int count, unsigned
 
 int gfd_zero_copy_gather_signal_presliced(const gfd_sg_entry* entries, int count, unsigned int* done_counter,
                                           uint64_t* done_word, uint64_t done_value, void* stream) {
-    return gfd_zero_copy_gather_signal(entries, count, done_counter, done_word, done_value, stream);
+    const int rc = gfd_zero_copy_gather_signal(entries, count, done_counter, done_word, done_value, stream);
+    g_zc_kind = "presliced";
+    return rc;
+}
+
+int gfd_zero_copy_gather_signal_equal(const void* entries, int count, unsigned int* done_counter, uint64_t* done_word,
+                                      uint64_t done_value, void* stream) {
+    const auto* e = static_cast<const gfd_sg_entry*>(entries);
+    const int rc = gfd_zero_copy_gather_signal(e, count, done_counter, done_word, done_value, stream);
+    g_zc_kind = "equal";
+    return rc;
 }
 
 int gfd_zero_copy_target_waves(void) {

@@ -423,6 +423,7 @@ int run_ragged(const std::string& path, uint32_t n, uint32_t nruns, int rounds, 
             if (p.submit_direct(sg.data(), (int)n) < 0) return 3;
             std::printf("zero-copy launches: %u\n", emu::zero_copy_launches() - zc0);
             std::printf("zero-copy records: %d\n", emu::zero_copy_records());
+            std::printf("zero-copy kind: %s\n", emu::zero_copy_kind());
             rc = check_image(dst, want, "ragged direct", rnd);
         }
     } else {

@@ -154,6 +154,19 @@ def test_direct_short_list_cut_for_the_waves_that_are_launched(poller_emu, waves
     assert all(least <= r <= most for r in records) and len(records) == 2, records
 
 
+@pytest.mark.parametrize("n,nruns,max_entry,kind", [(20, 1, 10000, "sliced"), (32, 1, 12000, "sliced"),
+                                                    (33, 1, 6000, "presliced"), (200, 100, 40000, "presliced"),
+                                                    (200, 100, 1, "equal"), (65, 65, 1, "equal"),
+                                                    (512, 200, 3000, "presliced"), (513, 200, 3000, "equal")])
+def test_direct_entry_lists_as_the_kernel_takes_them(poller_emu, n, nruns, max_entry, kind):
+    # Only a few uncut entries are left to the kernel's slices: from 33 on
+    # unequal entries get a wave each, equal or very many ones whole runs.
+    out = run(poller_emu, ["ragged", "direct", n, nruns, 2, 5],
+              env={"GFD_EMU_MAX_ENTRY": str(max_entry), "GFD_DIRECT_ZC_MIN_BYTES": "0"})
+    kinds = [l.split(": ")[1] for l in out.splitlines() if l.startswith("zero-copy kind:")]
+    assert kinds == [kind] * 2, kinds
+
+
 @pytest.mark.parametrize("zc_min,launches", [(0, 1), (64 << 20, 0)])
 def test_direct_zero_copy_minimum(poller_emu, zc_min, launches):
     # The one-run list of about 3 MiB: on the zero-copy route with no minimum,
