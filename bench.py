@@ -13,7 +13,8 @@ GB/s = bytes / (us * 1e3).
 
     python bench.py [--gpus 1] [--steps 50] [--warmup 15] [--only zc|direct|...]
 
-Prints ONE JSON line on stdout; progress goes to stderr.
+Prints ONE JSON line on stdout; progress, and the per-size tables that would
+make the line too long for its readers, go to stderr.
 """
 import argparse
 import ctypes
@@ -1350,6 +1351,28 @@ def flat_metric_fields(roofline, results, r_moe, r_worker=None):
             roofline[name + "_with_route_GBps"] = round(gbps(r_moe["bytes"], m["us_p50"] + route), 3)
 
 
+# Readers of the output keep its end only (16 KB), and a line that is cut does
+# not parse.  Per-size tables move to stderr, in this order, until it fits.
+LINE_CHARS = 15000
+DETAIL_KEYS = ("results_small", "results_direct_sizes", "results_short_lists", "results_timeline",
+               "results_helper_waves", "results_sessions")
+
+
+def output_line(result):
+    """(the JSON line, JSON of the tables that were moved out of it or None)."""
+    kept, moved = dict(result), {}
+
+    def dump(d):
+        return json.dumps(d, separators=(",", ":"))
+
+    for k in DETAIL_KEYS:
+        if len(dump(kept)) <= LINE_CHARS:
+            break
+        if kept.get(k):
+            moved[k] = kept.pop(k)
+    return dump(kept), dump(moved) if moved else None
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -1605,7 +1628,10 @@ def main():
                                                "num_ce_channels", "direct_chunk_bytes", "gather_slice_bytes")},
         "host": info,
     }
-    print(json.dumps(result), flush=True)
+    line, details = output_line(result)
+    if details:
+        print("details: " + details, file=sys.stderr, flush=True)
+    print(line, flush=True)
 
 
 if __name__ == "__main__":

@@ -1,6 +1,7 @@
 """CPU checks of bench.py's measurement helpers and its command-line contract:
 the parser behind roofline.traffic (rocprofv3 counter files), the summary of
 an SG session's per-list timeline, and the refusal of more than one GPU."""
+import json
 import os
 import subprocess
 import sys
@@ -62,6 +63,24 @@ def test_session_timeline_summary():
     assert s["last_exit_us"] == 95.0
     assert s["workgroup_last_landing_us"] == [70.0, 80.0, 90.0]
     assert s["claim_to_ready_mean_us"] == round((2 + 3 + 2 + 1) / 4, 2)
+
+
+def test_output_line_fits_its_readers():
+    """The line keeps the contract's fields whatever its size; the per-size
+    tables go elsewhere, whole, once it would be longer than a reader keeps."""
+    rows = [{"tokens": n, "queue": {"us_p50": 1.25, "sdma": {"e%d" % k: 0.5 for k in range(90)}}} for n in range(9)]
+    result = {"metric": "m", "value": 55.5, "unit": "GB/s", "ms_per_step": 0.6, "config": {"workload": "w"},
+              "roofline": {"f%d" % k: 1.0 / 3 for k in range(300)}, "results_small": rows,
+              "results_direct_sizes": rows[:1], "results_timeline": None}
+    line, details = bench.output_line(result)
+    assert "\n" not in line and len(line) <= bench.LINE_CHARS
+    kept = json.loads(line)
+    for k in ("metric", "value", "unit", "ms_per_step", "config", "roofline", "results_direct_sizes"):
+        assert kept[k] == result[k]
+    assert "results_small" not in kept and json.loads(details) == {"results_small": rows}
+    short = {"metric": "m", "value": 1.0, "results_small": rows[:1]}
+    line, details = bench.output_line(short)
+    assert json.loads(line) == short and details is None
 
 
 def test_bench_refuses_more_than_one_gpu():
