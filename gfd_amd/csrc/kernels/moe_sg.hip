@@ -222,8 +222,7 @@ __global__ __launch_bounds__(kListWaves * 64) void moe_route_kernel(const float*
     const int s0 = (int)blockIdx.x * share, s1 = min(s0 + share, num_tokens);
     for (int t = s0 + (int)threadIdx.x; t < s1; t += kListWaves * kWave)
         *reinterpret_cast<int2v*>(top2 + 2 * (size_t)t) = pairs[t];
-    place_rows<1>([&](int t) { return pairs[t]; }, num_tokens, num_experts, offsets,
-                                                    row_token);
+    place_rows<1>([&](int t) { return pairs[t]; }, num_tokens, num_experts, offsets, row_token);
 }
 
 // ------------------------------------------------------ gather + RMSNorm

@@ -413,8 +413,8 @@ int warp_spec_run(const void* cpu_src, void* gpu_dst, uint32_t total_tokens, uin
     auto p = s.get_launch_params();
     if (consumer == kWsRmsSin) p.grid = s.split_grid();  // a kSplitsChunks functor, as in launch()
     for (int it = 0; it < iters && rc == 0; it++) {
-        // launch() with the HIP events around the kernel alone: before_launch
-        // clears the signals with a blocking memset first.
+        // launch() with the HIP events around the kernel alone: the set-up
+        // kernel that before_launch puts on the stream goes ahead of them.
         s.before_launch(nullptr);
         (void)hipEventRecord(e0, nullptr);
         if (consumer == kWsTokenSum) {

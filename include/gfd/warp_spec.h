@@ -138,9 +138,10 @@ __device__ __forceinline__ int _wait_claimable(_TileSlot& sl, int epoch, uint32_
 }
 
 // Claim and compute token groups (G tokens) of chunk k of `tile`, the tile (or
-// part of one, S to a tile, K chunks and T tokens each) of slot `sl` at epoch `epoch` (its seq), until none is left.  The chunk must
-// have landed (the caller saw chunk_done[k] == P and made an acquire).  The
-// group that completes the chunk counts it in `done`.
+// part of one, S to a tile, K chunks and T tokens each) of slot `sl` at epoch
+// `epoch` (its seq), until none is left.  The chunk must have landed (the
+// caller saw chunk_done[k] == P and made an acquire).  The group that completes
+// the chunk counts it in `done`.
 template <typename ComputeFn>
 __device__ __forceinline__ void _compute_groups(_TileSlot& sl, int epoch, uint32_t tile, uint32_t k, uint32_t S,
                                                 uint32_t K, uint32_t T, uint32_t C, uint32_t G, uint32_t token_size,

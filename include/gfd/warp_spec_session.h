@@ -116,7 +116,8 @@ public:
         unsigned block;
     };
     LaunchParams get_launch_params() const;
-    // The grid launch() uses for a functor with kSplitsChunks: unless the
+    // The grid launch() uses for a functor with kSplitsChunks (size what such a
+    // functor indexes by workgroup with it): unless the
     // configuration sets num_blocks, few tiles are cut into parts of whole
     // chunks (warp_spec.h) for up to kSplitGrid workgroups.  Measured on
     // MI355X against one workgroup per tile (RMSNorm + sinf, kernel time): 64 x 4
