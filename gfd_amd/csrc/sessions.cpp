@@ -89,11 +89,18 @@ constexpr size_t report_offset(size_t bytes) { return (bytes + 63) & ~(size_t)63
 // ============================================================ WarpSpecSession
 
 void WarpSpecSession::release_spare_queues() {
-    std::lock_guard<std::mutex> lock(g_spare_mu);
-    for (; g_spares > 0; g_spares--) {
-        if (!still_there(g_spare[g_spares - 1])) continue;
-        gfd_hip_free(g_spare[g_spares - 1].signals);
-        gfd_hip_host_free(g_spare[g_spares - 1].tq);
+    SpareQueue all[kSpareQueues];
+    int n = 0;
+    {
+        std::lock_guard<std::mutex> lock(g_spare_mu);
+        while (g_spares > 0) all[n++] = g_spare[--g_spares];
+    }
+    // Not under the lock: a free waits for the device, whose kernels may wait
+    // for a thread that makes a session.
+    for (int i = 0; i < n; i++) {
+        if (!still_there(all[i])) continue;
+        gfd_hip_free(all[i].signals);
+        gfd_hip_host_free(all[i].tq);
     }
 }
 

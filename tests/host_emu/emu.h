@@ -56,6 +56,9 @@ void start_kernel(int device);
 bool kernel_runs(int device);
 // hipDeviceReset of the current device: what was allocated there is gone.
 void device_reset();
+// Called by every free of device memory, ahead of it (null: nothing): a free
+// waits for the device, and so for whatever its kernels wait for.
+void set_free_hook(void (*hook)());
 
 // Engine stall watchdog: an engine that has polled one dependency for longer
 // than this (GFD_EMU_STALL_MS, default 5000) prints what it waits on and ends

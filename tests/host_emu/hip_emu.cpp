@@ -26,6 +26,7 @@ constexpr int kMaxDevices = 4;
 int g_devices = 1;
 thread_local int t_device = 0;  // the thread's current device, as in HIP
 std::atomic<bool> g_kernel[kMaxDevices];
+std::atomic<void (*)()> g_free_hook{nullptr};
 
 std::mutex& reg_mu() {
     static std::mutex m;
@@ -66,6 +67,7 @@ void note_free(void* p) {
 void set_device_count(int n) { g_devices = n; }
 void start_kernel(int device) { g_kernel[device] = true; }
 bool kernel_runs(int device) { return g_kernel[device]; }
+void set_free_hook(void (*hook)()) { g_free_hook = hook; }
 void device_reset() {
     std::lock_guard<std::mutex> g(reg_mu());
     for (auto it = reg().begin(); it != reg().end();) {
@@ -186,6 +188,7 @@ int gfd_hip_malloc(void** p, size_t bytes) {
     return 0;
 }
 int gfd_hip_free(void* p) {
+    if (void (*hook)() = emu::g_free_hook.load()) hook();
     emu::note_free(p);
     std::free(p);
     return 0;

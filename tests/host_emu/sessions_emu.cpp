@@ -1,11 +1,15 @@
 // WarpSpecSession on the emulated runtime: its queue, and whom a destroyed
 // session leaves it to.  One scenario per run, named on the command line;
 // "pass" and status 0, or what went wrong and status 3.
+#include <chrono>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <future>
+#include <memory>
 #include <new>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "emu.h"
@@ -127,6 +131,29 @@ int run_device_reset() {
     return 0;
 }
 
+// release_spare_queues() waits in a free for a kernel that ends only once
+// another thread has made a session.
+bool g_made = false;
+std::thread g_other;
+void make_session_elsewhere() {
+    emu::set_free_hook(nullptr);
+    auto made = std::make_shared<std::promise<bool>>();
+    std::future<bool> f = made->get_future();
+    g_other = std::thread([made] {
+        WarpSpecSession s(config());
+        made->set_value(s.ok());
+    });
+    g_made = f.wait_for(std::chrono::seconds(5)) == std::future_status::ready && f.get();
+}
+int run_release() {
+    { WarpSpecSession a(config()); }
+    emu::set_free_hook(make_session_elsewhere);
+    WarpSpecSession::release_spare_queues();
+    if (g_other.joinable()) g_other.join();
+    REQUIRE(g_made);
+    return 0;
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -136,8 +163,9 @@ int main(int argc, char** argv) {
     if (what == "owner_device") rc = run_owner_device();
     if (what == "no_memory") rc = run_no_memory();
     if (what == "device_reset") rc = run_device_reset();
+    if (what == "release") rc = run_release();
     WarpSpecSession::release_spare_queues();
     if (rc == 0) std::printf("%s: pass\n", what.c_str());
-    if (rc == 4) std::fprintf(stderr, "usage: sessions_emu owner_device | no_memory | device_reset\n");
+    if (rc == 4) std::fprintf(stderr, "usage: sessions_emu owner_device | no_memory | device_reset | release\n");
     return rc;
 }

@@ -291,11 +291,12 @@ def test_queue_batches_through_the_zero_copy_worker(poller_emu, n, t, scattered,
     assert (jobs > 0) == want_jobs, out[-2000:]
 
 
-@pytest.mark.parametrize("what", ["owner_device", "no_memory", "device_reset"])
+@pytest.mark.parametrize("what", ["owner_device", "no_memory", "device_reset", "release"])
 def test_session_queues(poller_emu, what):
     """owner_device: a session destroyed with another device current waits for
     its own device's kernels before its queue is left to the next session.
     no_memory: a launch without the read-back kernel is synchronised by copies,
     and a session destroyed, where host memory has run out.
-    device_reset: queues that hipDeviceReset() took away are not handed on."""
+    device_reset: queues that hipDeviceReset() took away are not handed on.
+    release: spare queues are freed without keeping new sessions waiting."""
     run(os.path.join(os.path.dirname(poller_emu), "sessions_emu"), [what])
